@@ -836,7 +836,8 @@ struct gse_gseu_s {
 // Ewald direct space + self energy (CpuEwaldDirect.h:10-44)
 struct gse_ewald_direct_s {
   double sigma = 0, rcut = 0, ccelec = 332.0716, box[3] = {0, 0, 0};
-  DevBuf xofs, xlist, cell_of, counts, starts, fill, tmp, sidx, sx, partials, self2, mom;
+  DevBuf xofs, xlist, cell_of, rank, counts, starts, tmp, sidx, sx, sf, partials, q2,
+      erfcx;  // device copy of ew_erfcx_table
   bool have_excl = false;
   int n_excl_atoms = 0;
   hipStream_t stream = nullptr;
@@ -1984,8 +1985,8 @@ gse_status_t gse_ewald_direct_create(gse_ewald_direct_t* out, double sigma, doub
 
 gse_status_t gse_ewald_direct_destroy(gse_ewald_direct_t h) {
   if (!h) return GSE_SUCCESS;
-  for (DevBuf* b : {&h->xofs, &h->xlist, &h->cell_of, &h->counts, &h->starts, &h->fill, &h->tmp,
-                    &h->sidx, &h->sx, &h->partials, &h->self2, &h->mom})
+  for (DevBuf* b : {&h->xofs, &h->xlist, &h->cell_of, &h->rank, &h->counts, &h->starts, &h->tmp,
+                    &h->sidx, &h->sx, &h->sf, &h->partials, &h->q2, &h->erfcx})
     b->release();
   delete h;
   return GSE_SUCCESS;
@@ -2053,44 +2054,37 @@ gse_status_t gse_ewald_direct_calc_force_energy(gse_ewald_direct_t h, int n, con
     return fail(GSE_ERROR_INVALID_VALUE, "the exclusion list covers %d atoms, the call %d",
                 h->n_excl_atoms, n);
   EwCells c;
-  c.ncell = 1;
-  for (int a = 0; a < 3; a++) {
-    c.box[a] = h->box[a];
-    int nc = (int)std::floor(h->box[a] / h->rcut);
-    if (nc > 128) nc = 128;
-    c.nc[a] = nc >= 3 ? nc : 1;
-    c.ncell *= c.nc[a];
-  }
+  ew_cells_make(h->box, h->rcut, n, &c);
   EwPair p;
   p.rcut2 = h->rcut * h->rcut;
   p.ccelec = h->ccelec;
   p.inv_sqrt2sigma = 1.0 / (std::sqrt(2.0) * h->sigma);
   p.inv_2sigmasq = 1.0 / (2.0 * h->sigma * h->sigma);
   p.two_sqrtpi = 2.0 / std::sqrt(M_PI);
+  ew_filter_make(c, &p);
   const size_t n1 = (size_t)(n > 0 ? n : 1);
-  GSECHK(h->cell_of.ensure(sizeof(int) * n1));
-  GSECHK(h->tmp.ensure(sizeof(int) * n1));
-  GSECHK(h->sidx.ensure(sizeof(int) * n1));
+  for (DevBuf* b : {&h->cell_of, &h->rank, &h->tmp, &h->sidx}) GSECHK(b->ensure(sizeof(int) * n1));
   GSECHK(h->sx.ensure(4 * sizeof(double) * n1));
+  GSECHK(h->sf.ensure(4 * sizeof(float) * n1));
   GSECHK(h->counts.ensure(sizeof(int) * c.ncell));
-  GSECHK(h->starts.ensure(sizeof(int) * c.ncell));
-  GSECHK(h->fill.ensure(sizeof(int) * c.ncell));
-  GSECHK(h->partials.ensure(sizeof(double) * c.ncell));
-  GSECHK(h->mom.ensure(sizeof(double) * kRedBlocks * 2));
-  GSECHK(h->self2.ensure(sizeof(double) * 2));
+  GSECHK(h->starts.ensure(sizeof(int) * (c.ncell + 1)));
+  GSECHK(h->partials.ensure(sizeof(double) * n1));
+  GSECHK(h->q2.ensure(sizeof(double) * kEwCountBlocks));
+  if (!h->erfcx.p) {
+    GSECHK(h->erfcx.ensure(ew_erfcx_bytes()));
+    HIPCHK(hipMemcpy(h->erfcx.p, ew_erfcx_table(), ew_erfcx_bytes(), hipMemcpyHostToDevice));
+  }
   hipStream_t s = h->stream;
-  HIPCHK(launch_ew_cells(xyzq, n, c, h->cell_of.as<int>(), h->counts.as<int>(),
-                         h->starts.as<int>(), h->fill.as<int>(), h->tmp.as<int>(),
-                         h->sidx.as<int>(), h->sx.p, s));
-  HIPCHK(launch_ew_force(c, p, h->starts.as<int>(), h->counts.as<int>(), h->sidx.as<int>(),
-                         h->sx.p, h->have_excl ? h->xofs.as<int>() : nullptr,
-                         h->have_excl ? h->xlist.as<int>() : nullptr, fx, fy, fz,
-                         h->partials.as<double>(), s));
+  HIPCHK(launch_ew_cells(xyzq, n, c, h->rcut, h->cell_of.as<int>(), h->rank.as<int>(),
+                         h->counts.as<int>(), h->starts.as<int>(), h->tmp.as<int>(),
+                         h->sidx.as<int>(), h->sx.p, h->sf.p, h->q2.as<double>(), s));
+  HIPCHK(launch_ew_force(n, c, p, h->starts.as<int>(), h->sidx.as<int>(), h->sx.p, h->sf.p,
+                         h->have_excl ? h->xofs.as<int>() : nullptr,
+                         h->have_excl ? h->xlist.as<int>() : nullptr, h->erfcx.as<double>(), fx, fy,
+                         fz, h->partials.as<double>(), s));
   // self energy -ccelec sum q^2 / sqrt(2 pi sigma^2) (CpuEwaldDirect.cpp:124-128)
-  HIPCHK(launch_charge_moments(true, xyzq, n, h->mom.as<double>(), s));
-  HIPCHK(launch_corrections_finalize(h->mom.as<double>(), kRedBlocks, h->sigma, 1.0, 1.0, 1.0,
-                                     h->ccelec, h->self2.as<double>(), s));
-  HIPCHK(launch_ew_finalize(h->partials.as<double>(), c.ncell, h->self2.as<double>(), energy, s));
+  HIPCHK(launch_ew_finalize(h->partials.as<double>(), n, h->q2.as<double>(),
+                            -h->ccelec / std::sqrt(2.0 * M_PI * h->sigma * h->sigma), energy, s));
   return GSE_SUCCESS;
 }
 

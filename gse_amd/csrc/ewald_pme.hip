@@ -18,14 +18,17 @@
 //
 // Ewald direct space (CpuEwaldDirect.cpp:45-131):
 //   k_ew_cell_count / k_ew_scan / k_ew_scatter / k_ew_sort
-//                   particles into cells of edge >= rcut, each cell's list in
-//                   ascending particle index (deterministic order)
-//   k_ew_force      one workgroup per cell: four lanes share one particle
-//                   (each a quarter of its neighbours, summed across the four
-//                   in a fixed order), neighbour cells are staged through
-//                   LDS, the pair term of
-//                   the reference is evaluated with its operand order and
-//                   minimum-image loops; FP64 energy partial per cell
+//                   particles into cells, each cell's list in ascending
+//                   particle index (deterministic order); partial sums of q^2
+//   k_ew_force      one wave per group of particles: candidates of the cells
+//                   within reach pass a 32-bit distance filter into a queue,
+//                   full queues are evaluated in FP64 with the reference's
+//                   operand order and minimum-image loops
+//   k_ew_finalize   energy of the groups and the self term
+#include <algorithm>
+#include <cmath>
+#include <vector>
+
 #include <math.h>
 
 #include "gse_device.h"
@@ -452,78 +455,97 @@ hipError_t launch_pme_gather(bool ct_dbl, bool at_dbl, int order, const void* xy
 // ---------------------------------------------------------------------------
 // Ewald direct space
 // ---------------------------------------------------------------------------
-// cell of one coordinate: wrapped into [0, L), cells of edge L/nc
-__device__ __forceinline__ int ew_cell1(double x, double L, int nc) {
-  double w = x - L * floor(x / L);
-  if (!(w >= 0.0 && w < L)) return 0;
+// one coordinate wrapped into [0, L) (NaN for a non-finite one) and its cell
+// of edge L/nc
+__device__ __forceinline__ double ew_wrap(double x, double L) {
+  const double w = x - L * floor(x / L);
+  return w >= L || w < 0.0 ? 0.0 : w;
+}
+__device__ __forceinline__ int ew_cell1(double w, double L, int nc) {
+  if (!(w >= 0.0)) return 0;
   const int c = (int)(w * ((double)nc / L));
   return c < nc ? c : nc - 1;
 }
 
-__global__ void k_ew_cell_count(const P4<double>* __restrict__ xyzq, int n, EwCells c,
-                                int* __restrict__ cell_of, int* __restrict__ counts) {
+// Cell and arrival rank of every particle, and the partial sums of q^2 for
+// the self term (one per workgroup, fixed order).  The cells hold about six
+// particles, so few atomics meet on one counter (a cell of edge rcut holds
+// ninety, and 48,000 atomics on 512 counters took 26 us).
+__global__ __launch_bounds__(256) void k_ew_cell_count(const P4<double>* __restrict__ xyzq, int n,
+                                                       EwCells c, int* __restrict__ cell_of,
+                                                       int* __restrict__ rank,
+                                                       int* __restrict__ counts,
+                                                       double* __restrict__ q2) {
+  __shared__ double sh[4];
+  double acc = 0.0;
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     const P4<double> r = xyzq[i];
-    const int cx = ew_cell1(r.x, c.box[0], c.nc[0]), cy = ew_cell1(r.y, c.box[1], c.nc[1]),
-              cz = ew_cell1(r.z, c.box[2], c.nc[2]);
+    const int cx = ew_cell1(ew_wrap(r.x, c.box[0]), c.box[0], c.nc[0]),
+              cy = ew_cell1(ew_wrap(r.y, c.box[1]), c.box[1], c.nc[1]),
+              cz = ew_cell1(ew_wrap(r.z, c.box[2]), c.box[2], c.nc[2]);
     const int cell = cx + (cy + cz * c.nc[1]) * c.nc[0];
     cell_of[i] = cell;
-    atomicAdd(&counts[cell], 1);
+    rank[i] = atomicAdd(&counts[cell], 1);
+    acc += r.w * r.w;
   }
-}
-
-// exclusive scan of the cell counts by one workgroup; fill[] cleared
-__global__ __launch_bounds__(1024) void k_ew_scan(const int* __restrict__ counts, int ncell,
-                                                  int* __restrict__ starts,
-                                                  int* __restrict__ fill) {
-  __shared__ int sh[1024];
-  __shared__ int carry;
-  if (threadIdx.x == 0) carry = 0;
+  const double w = wave_sum(acc);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = w;
   __syncthreads();
-  for (int base = 0; base < ncell; base += 1024) {
-    const int i = base + threadIdx.x;
-    const int v = i < ncell ? counts[i] : 0;
-    sh[threadIdx.x] = v;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-      const int t = threadIdx.x >= off ? sh[threadIdx.x - off] : 0;
-      __syncthreads();
-      sh[threadIdx.x] += t;
-      __syncthreads();
-    }
-    if (i < ncell) {
-      starts[i] = carry + sh[threadIdx.x] - v;
-      fill[i] = 0;
-    }
-    __syncthreads();
-    if (threadIdx.x == 1023) carry += sh[1023];
-    __syncthreads();
-  }
+  if (threadIdx.x == 0) q2[blockIdx.x] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
 }
 
-__global__ void k_ew_scatter(int n, const int* __restrict__ cell_of,
-                             const int* __restrict__ starts, int* __restrict__ fill,
-                             int* __restrict__ tmp) {
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const int c = cell_of[i];
-    tmp[starts[c] + atomicAdd(&fill[c], 1)] = i;
+// exclusive scan of the cell counts by one workgroup, consecutive cells per
+// thread; starts[ncell] = all particles
+__global__ __launch_bounds__(1024) void k_ew_scan(const int* __restrict__ counts, int ncell,
+                                                  int* __restrict__ starts) {
+  __shared__ int sh[16];
+  const int per = (ncell + 1023) / 1024;
+  const int i0 = min((int)threadIdx.x * per, ncell), i1 = min(i0 + per, ncell);
+  int sum = 0;
+  for (int i = i0; i < i1; i++) sum += counts[i];
+  int v = sum;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int t = __shfl_up(v, d, kWave);
+    if ((int)(threadIdx.x & 63) >= d) v += t;
   }
+  if ((threadIdx.x & 63) == 63) sh[threadIdx.x >> 6] = v;
+  __syncthreads();
+  int run = v - sum;
+  for (int w = 0; w < (int)(threadIdx.x >> 6); w++) run += sh[w];
+  for (int i = i0; i < i1; i++) {
+    starts[i] = run;
+    run += counts[i];
+  }
+  if (threadIdx.x == 1023) starts[ncell] = run;
 }
 
-// each cell's particles in ascending index: the rank of a slot is the number
-// of the cell's particles with a smaller index
-__global__ void k_ew_sort(int n, const int* __restrict__ cell_of, const int* __restrict__ starts,
-                          const int* __restrict__ counts, const int* __restrict__ tmp,
+__global__ void k_ew_scatter(int n, const int* __restrict__ cell_of, const int* __restrict__ rank,
+                             const int* __restrict__ starts, int* __restrict__ tmp) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+    tmp[starts[cell_of[i]] + rank[i]] = i;
+}
+
+// Each cell's particles in ascending index (deterministic): the rank of a
+// slot is the number of the cell's particles with a smaller index.  sf holds
+// the wrapped position in units of rcut, rounded to 32 bits, and the cell,
+// for the distance filter of k_ew_force.
+__global__ void k_ew_sort(int n, EwCells c, double inv_rcut, const int* __restrict__ cell_of,
+                          const int* __restrict__ starts, const int* __restrict__ tmp,
                           const P4<double>* __restrict__ xyzq, int* __restrict__ sidx,
-                          P4<double>* __restrict__ sx) {
+                          P4<double>* __restrict__ sx, P4<float>* __restrict__ sf) {
   for (int s = blockIdx.x * blockDim.x + threadIdx.x; s < n; s += gridDim.x * blockDim.x) {
     const int i = tmp[s];
-    const int c = cell_of[i];
-    const int st = starts[c], cnt = counts[c];
-    int rank = 0;
-    for (int k = 0; k < cnt; k++) rank += tmp[st + k] < i;
-    sidx[st + rank] = i;
-    sx[st + rank] = xyzq[i];
+    const int cell = cell_of[i];
+    const int st = starts[cell], en = starts[cell + 1];
+    int k = st;
+    for (int t = st; t < en; t++) k += tmp[t] < i;
+    const P4<double> r = xyzq[i];
+    sidx[k] = i;
+    sx[k] = r;
+    sf[k] = P4<float>{(float)(ew_wrap(r.x, c.box[0]) * inv_rcut),
+                      (float)(ew_wrap(r.y, c.box[1]) * inv_rcut),
+                      (float)(ew_wrap(r.z, c.box[2]) * inv_rcut), __int_as_float(cell)};
   }
 }
 
@@ -537,153 +559,388 @@ __device__ __forceinline__ double ew_image(double d, double L, double h) {
   return d;
 }
 
-constexpr int kEwBlock = 128;  // particles of a cell per pass
-constexpr int kEwSplit = 4;    // threads per particle, each a quarter of the neighbours
-constexpr int kEwThreads = kEwBlock * kEwSplit;
+// the same value for the common case, at most one step either way, without
+// loops; `far` collects coordinates that need them
+__device__ __forceinline__ double ew_image1(double d, double L, double h, bool& far) {
+  double v = d < -h ? d + L : d;
+  v = v > h ? v - L : v;
+  far = far || !(v >= -h && v <= h);
+  return v;
+}
 
-// One workgroup per cell; kEwSplit consecutive lanes share one particle of
-// the cell and take every kEwSplit-th neighbour of each staged neighbour
-// cell, and their sums are added across the four lanes in a fixed order.
-__global__ __launch_bounds__(kEwThreads) void k_ew_force(
-    EwCells c, EwPair pr, const int* __restrict__ starts, const int* __restrict__ counts,
-    const int* __restrict__ sidx, const P4<double>* __restrict__ sx,
-    const int* __restrict__ xofs, const int* __restrict__ xlist, double* __restrict__ gx,
-    double* __restrict__ gy, double* __restrict__ gz, double* __restrict__ partials) {
-  __shared__ P4<double> shp[kEwBlock];
-  __shared__ int shi[kEwBlock];
-  __shared__ double she[kEwThreads / 64];
-  const int cell = blockIdx.x;
-  const int cx = cell % c.nc[0], cy = (cell / c.nc[0]) % c.nc[1], cz = cell / (c.nc[0] * c.nc[1]);
-  const int st = starts[cell], cnt = counts[cell];
-  const int lo0 = c.nc[0] >= 3 ? -1 : 0, lo1 = c.nc[1] >= 3 ? -1 : 0, lo2 = c.nc[2] >= 3 ? -1 : 0;
-  const int slot = threadIdx.x / kEwSplit, sp = threadIdx.x % kEwSplit;
-  double esum = 0.0;
-  for (int base = 0; base < cnt; base += kEwBlock) {
-    const int t = base + slot;
-    const bool own = t < cnt;
-    const int a = own ? sidx[st + t] : -1;
-    P4<double> pa{0.0, 0.0, 0.0, 0.0};
-    int x0 = 0, x1 = 0;
-    if (own) {
-      pa = sx[st + t];
-      if (xofs) {
-        x0 = xofs[a];
-        x1 = xofs[a + 1];
+// erfc(x) = exp(-x^2) erfcx(x), and the pair term needs that exponential
+// anyway: erfcx is a polynomial of degree 11 about the centre of x's
+// interval (width 1/4 below 8, 1 up to 27, where erfc underflows), fitted at
+// Chebyshev nodes in extended precision; its error is below one unit in the
+// last place (2.1e-16), at 12 multiply-adds where the library's erfc takes
+// about 150 FP64 instructions.
+constexpr int kErfcxRows = 51, kErfcxDeg = 11, kErfcxPitch = 14;  // doubles a row, 16-byte rows
+
+const double* ew_erfcx_table() {
+  static const std::vector<double> table = [] {
+    typedef long double L;
+    const L pi = 3.14159265358979323846264338327950288L;
+    constexpr int n = kErfcxDeg + 1;
+    std::vector<double> out(kErfcxRows * kErfcxPitch, 0.0);
+    for (int row = 0; row < kErfcxRows; row++) {
+      const L c = row < 32 ? (row + 0.5L) * 0.25L : row - 24 + 0.5L, h = row < 32 ? 0.125L : 0.5L;
+      L f[n], mono[n] = {}, t0[n] = {}, t1[n] = {};
+      for (int k = 0; k < n; k++) {
+        const L x = c + h * cosl(pi * (k + 0.5L) / n);
+        f[k] = erfcl(x) * expl(x * x);
+      }
+      // sum of the Chebyshev polynomials as powers of u = (x - c) / h
+      t0[0] = 1.0L;
+      t1[1] = 1.0L;
+      for (int j = 0; j < n; j++) {
+        L a = 0.0L;
+        for (int k = 0; k < n; k++) a += f[k] * cosl(pi * j * (k + 0.5L) / n);
+        a *= (j == 0 ? 1.0L : 2.0L) / n;
+        for (int k = 0; k < n; k++) mono[k] += a * t0[k];
+        for (int k = n - 1; k >= 0; k--) {  // (T_j, T_j+1) -> (T_j+1, T_j+2)
+          const L next = (k > 0 ? 2.0L * t1[k - 1] : 0.0L) - t0[k];
+          t0[k] = next;
+        }
+        for (int k = 0; k < n; k++) std::swap(t0[k], t1[k]);
+      }
+      L p = 1.0L;
+      for (int k = 0; k < n; k++, p *= h) out[row * kErfcxPitch + k] = (double)(mono[k] / p);
+    }
+    return out;
+  }();
+  return table.data();
+}
+
+size_t ew_erfcx_bytes() { return sizeof(double) * kErfcxRows * kErfcxPitch; }
+
+__device__ __forceinline__ double ew_erfcx(const double* tab, double x) {
+  x = fmin(x, 27.0);  // the exponential is zero from there on
+  const bool fine = x < 8.0;
+  const int cell = (int)(fine ? 4.0 * x : x);
+  const double mid = (double)cell + 0.5, d = x - (fine ? 0.25 * mid : mid);
+  const double* t = tab + min(fine ? cell : cell + 24, kErfcxRows - 1) * kErfcxPitch;
+  double v = t[kErfcxDeg];
+#pragma unroll
+  for (int k = kErfcxDeg - 1; k >= 0; k--) v = __builtin_fma(v, d, t[k]);
+  return v;
+}
+
+// Force and energy of one particle per wave, in the order of the cells.
+//
+// The pair term costs about 150 FP64 instructions and one candidate in three
+// is within rcut, so testing and evaluating in one loop runs the pair term
+// with a third of the lanes.  Here the wave takes 64 candidates at a time,
+// tests them in 32 bits (rcut widened by the rounding of the positions, so no
+// pair is lost), and appends the survivors to a queue in LDS; 64 of them are
+// evaluated with all lanes in FP64 (the reference's operand order and strict
+// r2 < rcut2 test on the exact positions).  Two and four particles per wave,
+// sharing the candidate loads, were no faster (293 against 288 us) for want
+// of waves.
+// Candidates are the cells within reach: rows of cells along x are one
+// contiguous range of the sorted particles (two where the row wraps), found
+// by one lane per range and cut to the sphere around the particle.  Cells of
+// rcut/4 x rcut/2 x rcut/2 make a row range at most about 50 particles of
+// liquid water, one batch of 64; cells of edge rcut take 2,500 candidates.
+// On the 48,000-charge box at rcut 9 (14.6 M pair terms): 240 us, 110 M VALU
+// instructions (180 us of issue), against 1475 us with one loop over the 27
+// cells of edge rcut around each; 3,000 charges 31 us.
+// Each lane adds its terms in the order of the cells, then the lanes are
+// added in a fixed order: no atomics, the same bits on every run.
+constexpr int kEwWaves = 4;
+template <bool FOLD>
+__global__ __launch_bounds__(64 * kEwWaves) void k_ew_force(
+    int n, EwCells c, EwPair pr, const int* __restrict__ starts, const int* __restrict__ sidx,
+    const P4<double>* __restrict__ sx, const P4<float>* __restrict__ sf,
+    const int* __restrict__ xofs, const int* __restrict__ xlist,
+    const double* __restrict__ erfcx, double* __restrict__ gx, double* __restrict__ gy,
+    double* __restrict__ gz, double* __restrict__ partials) {
+  __shared__ int queue[kEwWaves][128];
+  __shared__ alignas(16) double ertab[kErfcxRows * kErfcxPitch];
+  for (int k = threadIdx.x; k < kErfcxRows * kErfcxPitch; k += 64 * kEwWaves) ertab[k] = erfcx[k];
+  __syncthreads();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int islot = blockIdx.x * kEwWaves + wave;
+  if (islot >= n) return;  // no barrier follows
+  int* q = queue[wave];
+
+  const P4<float> pf = sf[islot];
+  const int cell = __builtin_amdgcn_readfirstlane(__float_as_int(pf.w));
+  const int a = sidx[islot];
+  const P4<double> pa = sx[islot];
+  // the first exclusions stay in registers (a water atom has two)
+  const int ex0 = xofs ? xofs[a] : 0, ex1 = xofs ? xofs[a + 1] : 0;
+  int ex[4];
+#pragma unroll
+  for (int x = 0; x < 4; x++) ex[x] = ex0 + x < ex1 ? xlist[ex0 + x] : -1;
+
+  // candidate ranges: lane 2r + part holds part 0 or 1 of row r's range.  An
+  // axis whose cells all lie within reach is visited once and its distances
+  // folded to the nearest image; the others carry the image's shift.
+  const bool ally = FOLD && c.nc[1] <= 2 * c.reach[1] + 1,
+             allz = FOLD && c.nc[2] <= 2 * c.reach[2] + 1;
+  const int nyr = ally ? c.nc[1] : 2 * c.reach[1] + 1;
+  const int nzr = allz ? c.nc[2] : 2 * c.reach[2] + 1;
+  int s = 0, t = 0;
+  float hx = 0.f, hy = 0.f, hz = 0.f;  // added to the candidate's position
+  bool whole = false;
+  {
+    const int r = lane >> 1, part = lane & 1;
+    if (r < nyr * nzr) {
+      const int row = cell / c.nc[0];
+      int y = r % nyr, z = r / nyr;
+      float d2 = 0.f;  // squared distance of the particle to the row
+      if (!ally) {
+        y += row % c.nc[1] - c.reach[1];
+        const float e = c.len[1] / (float)c.nc[1], lo = e * (float)y;
+        const float d = fmaxf(fmaxf(lo - pf.y, pf.y - (lo + e)) - pr.slack, 0.f);
+        d2 += d * d;
+        if (y < 0) {
+          y += c.nc[1];
+          hy = -c.len[1];
+        } else if (y >= c.nc[1]) {
+          y -= c.nc[1];
+          hy = c.len[1];
+        }
+      }
+      if (!allz) {
+        z += row / c.nc[1] - c.reach[2];
+        const float e = c.len[2] / (float)c.nc[2], lo = e * (float)z;
+        const float d = fmaxf(fmaxf(lo - pf.z, pf.z - (lo + e)) - pr.slack, 0.f);
+        d2 += d * d;
+        if (z < 0) {
+          z += c.nc[2];
+          hz = -c.len[2];
+        } else if (z >= c.nc[2]) {
+          z -= c.nc[2];
+          hz = c.len[2];
+        }
+      }
+      int x0 = 0, x1 = -1;
+      if (d2 <= pr.filter2) {  // false for a particle at a position that is not finite
+        const float w = sqrtf(pr.filter2 - d2) + pr.slack, ie = (float)c.nc[0] / c.len[0];
+        const int lo = (int)floorf((pf.x - w) * ie), hi = (int)floorf((pf.x + w) * ie);
+        whole = FOLD && hi - lo + 1 >= c.nc[0];
+        if (whole) {
+          if (part == 0) x1 = c.nc[0] - 1;
+        } else if (lo < 0) {
+          x0 = part ? 0 : lo + c.nc[0];
+          x1 = part ? hi : c.nc[0] - 1;
+          hx = part ? 0.f : -c.len[0];
+        } else if (hi >= c.nc[0]) {
+          x0 = part ? 0 : lo;
+          x1 = part ? hi - c.nc[0] : c.nc[0] - 1;
+          hx = part ? c.len[0] : 0.f;
+        } else if (part == 0) {
+          x0 = lo;
+          x1 = hi;
+        }
+      }
+      if (x1 >= x0) {
+        const int rc = (y + z * c.nc[1]) * c.nc[0];
+        s = starts[rc + x0];
+        t = starts[rc + x1 + 1];
       }
     }
-    double g0 = 0.0, g1 = 0.0, g2 = 0.0, e = 0.0;
-    for (int dz = lo2; dz <= -lo2; dz++)
-      for (int dy = lo1; dy <= -lo1; dy++)
-        for (int dx = lo0; dx <= -lo0; dx++) {
-          const int nx = (cx + dx + c.nc[0]) % c.nc[0], ny = (cy + dy + c.nc[1]) % c.nc[1],
-                    nz = (cz + dz + c.nc[2]) % c.nc[2];
-          const int nb = nx + (ny + nz * c.nc[1]) * c.nc[0];
-          const int nst = starts[nb], ncnt = counts[nb];
-          for (int kb = 0; kb < ncnt; kb += kEwBlock) {
-            __syncthreads();
-            if ((int)threadIdx.x < kEwBlock && kb + (int)threadIdx.x < ncnt) {
-              shp[threadIdx.x] = sx[nst + kb + threadIdx.x];
-              shi[threadIdx.x] = sidx[nst + kb + threadIdx.x];
-            }
-            __syncthreads();
-            const int m = min(kEwBlock, ncnt - kb);
-            if (!own) continue;
-            for (int k = sp; k < m; k += kEwSplit) {
-              const int b = shi[k];
-              if (b == a) continue;
-              const P4<double> pb = shp[k];
-              const double ddx = ew_image(pa.x - pb.x, c.box[0], 0.5 * c.box[0]);
-              const double ddy = ew_image(pa.y - pb.y, c.box[1], 0.5 * c.box[1]);
-              const double ddz = ew_image(pa.z - pb.z, c.box[2], 0.5 * c.box[2]);
-              const double r2 = ddx * ddx + ddy * ddy + ddz * ddz;
-              if (!(r2 < pr.rcut2)) continue;
-              bool excl = false;
-              for (int q = x0; q < x1; q++) excl = excl || xlist[q] == b;
-              if (excl) continue;
-              // qq = (q_j ccelec) q_i with j the smaller index (:69, :101)
-              const double qq = a < b ? (pa.w * pr.ccelec) * pb.w : (pb.w * pr.ccelec) * pa.w;
-              const double r = sqrt(r2);
-              const double erfcval = erfc(r * pr.inv_sqrt2sigma);
-              const double expval = exp(-r2 * pr.inv_2sigmasq);
-              const double f = -qq * (pr.two_sqrtpi * pr.inv_sqrt2sigma * expval + erfcval / r) / r2;
-              g0 += f * ddx;
-              g1 += f * ddy;
-              g2 += f * ddz;
-              e += qq * erfcval / r;
-            }
-          }
-        }
-    // the particle's four partial sums, added in a fixed order (xor 1, then
-    // xor 2: every lane of the four ends with the same value)
-#pragma unroll
-    for (int m = 1; m < kEwSplit; m <<= 1) {
-      g0 += __shfl_xor(g0, m, kWave);
-      g1 += __shfl_xor(g1, m, kWave);
-      g2 += __shfl_xor(g2, m, kWave);
-    }
-    if (own && sp == 0) {
-      gx[a] = g0;
-      gy[a] = g1;
-      gz[a] = g2;
-    }
-    esum += e;
   }
-  // every pair was met from both ends: half of the sum per cell
-  const double w = wave_sum(esum);
-  if ((threadIdx.x & 63) == 0) she[threadIdx.x >> 6] = w;
+  unsigned long long pieces = __ballot(t > s);
+  const float fy = ally ? 1.f / c.len[1] : 0.f, fz = allz ? 1.f / c.len[2] : 0.f;
+  const float fx = FOLD ? (whole ? 1.f / c.len[0] : 0.f) : 0.f;
+
+  int k = 0, kend = 0, held = 0;
+  float px = 0.f, py = 0.f, pz = 0.f, pfx = 0.f;
+  P4<float> cand{0.f, 0.f, 0.f, 0.f};
+  bool have = false;
+  auto fetch = [&]() {
+    k += 64;
+    have = true;
+    if (k >= kend) {
+      have = pieces != 0ull;
+      if (have) {
+        const int p = __builtin_ctzll(pieces);
+        pieces &= pieces - 1ull;
+        k = __builtin_amdgcn_readlane(s, p);
+        kend = __builtin_amdgcn_readlane(t, p);
+        px = readlane(hx, p);
+        py = readlane(hy, p);
+        pz = readlane(hz, p);
+        if (FOLD) pfx = readlane(fx, p);
+      }
+    }
+    if (have) cand = sf[min(k + lane, kend - 1)];
+  };
+  double g0 = 0.0, g1 = 0.0, g2 = 0.0, e = 0.0;
+  fetch();
+  for (;;) {
+    const bool more = have;
+    if (more) {
+      const int slot = k + lane;
+      const bool in = slot < kend;
+      float dx = pf.x - (cand.x + px), dy = pf.y - (cand.y + py), dz = pf.z - (cand.z + pz);
+      if (FOLD) {
+        dx -= c.len[0] * rintf(dx * pfx);
+        dy -= c.len[1] * rintf(dy * fy);
+        dz -= c.len[2] * rintf(dz * fz);
+      }
+      fetch();  // the next candidates load while these are tested
+      const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
+      const bool hit = in & (r2 < pr.filter2);
+      const unsigned long long m = __ballot(hit);
+      const unsigned at = __builtin_amdgcn_mbcnt_hi(
+          (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, (unsigned)held));
+      if (hit) q[at] = slot;
+      held += __popcll(m);
+    }
+    // 64 fill the wave; after the last candidates, all that is left
+    if (held < 64 && (more || held == 0)) {
+      if (!more) break;
+      continue;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (lane < held) {
+      const int sl = q[lane];
+      const P4<double> pb = sx[sl];
+      const int b = sidx[sl];
+      bool far = false;
+      double ddx = ew_image1(pa.x - pb.x, c.box[0], 0.5 * c.box[0], far);
+      double ddy = ew_image1(pa.y - pb.y, c.box[1], 0.5 * c.box[1], far);
+      double ddz = ew_image1(pa.z - pb.z, c.box[2], 0.5 * c.box[2], far);
+      if (__builtin_expect(far, 0)) {
+        ddx = ew_image(pa.x - pb.x, c.box[0], 0.5 * c.box[0]);
+        ddy = ew_image(pa.y - pb.y, c.box[1], 0.5 * c.box[1]);
+        ddz = ew_image(pa.z - pb.z, c.box[2], 0.5 * c.box[2]);
+      }
+      const double r2 = ddx * ddx + ddy * ddy + ddz * ddz;
+      bool ok = r2 < pr.rcut2 && sl != islot;
+#pragma unroll
+      for (int x = 0; x < 4; x++) ok = ok && ex[x] != b;
+      for (int x = ex0 + 4; x < ex1; x++) ok = ok && xlist[x] != b;
+      if (ok) {
+        // qq = (q_j ccelec) q_i with j the smaller index (:69, :101)
+        const double qq = a < b ? (pa.w * pr.ccelec) * pb.w : (pb.w * pr.ccelec) * pa.w;
+        const double r = sqrt(r2);
+        const double expval = exp(-r2 * pr.inv_2sigmasq);
+        const double er = expval * ew_erfcx(ertab, r * pr.inv_sqrt2sigma) / r;
+        const double f = -qq * (pr.two_sqrtpi * pr.inv_sqrt2sigma * expval + er) / r2;
+        g0 += f * ddx;
+        g1 += f * ddy;
+        g2 += f * ddz;
+        e += qq * er;
+      }
+    }
+    // the queue's tail moves to its front
+    held = max(held - 64, 0);
+    const int tail = lane < held ? q[64 + lane] : 0;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (lane < held) q[lane] = tail;
+  }
+  g0 = wave_total(g0);
+  g1 = wave_total(g1);
+  g2 = wave_total(g2);
+  e = wave_total(e);
+  if (lane == 0) {
+    gx[a] = g0;
+    gy[a] = g1;
+    gz[a] = g2;
+    // every pair is met from both ends
+    partials[islot] = 0.5 * e;
+  }
+}
+
+// energy = sum of the particles' partials (sorted order) + the self term
+// -ccelec sum q^2 / sqrt(2 pi sigma^2) (CpuEwaldDirect.cpp:124-128)
+__global__ __launch_bounds__(1024) void k_ew_finalize(const double* __restrict__ partials,
+                                                      int n, const double* __restrict__ q2,
+                                                      int nq2, double self, double* energy) {
+  __shared__ double she[16], shq[16];
+  double s = 0.0, w = 0.0;
+  for (int i = threadIdx.x; i < n; i += 1024) s += partials[i];
+  for (int i = threadIdx.x; i < nq2; i += 1024) w += q2[i];
+  s = wave_sum(s);
+  w = wave_sum(w);
+  if ((threadIdx.x & 63) == 0) {
+    she[threadIdx.x >> 6] = s;
+    shq[threadIdx.x >> 6] = w;
+  }
   __syncthreads();
   if (threadIdx.x == 0) {
-    double tot = 0.0;
-    for (int k = 0; k < kEwThreads / 64; k++) tot += she[k];
-    partials[cell] = 0.5 * tot;
+    double te = 0.0, tq = 0.0;
+    for (int k = 0; k < 16; k++) {
+      te += she[k];
+      tq += shq[k];
+    }
+    energy[0] = te + self * tq;
   }
 }
 
-// energy = sum of the cell partials (cell order) + the self term
-__global__ void k_ew_finalize(const double* __restrict__ partials, int ncell,
-                              const double* __restrict__ self2, double* energy) {
-  __shared__ double sh[256];
-  double s = 0.0;
-  for (int i = threadIdx.x; i < ncell; i += 256) s += partials[i];
-  sh[threadIdx.x] = s;
-  __syncthreads();
-  for (int off = 128; off >= 1; off >>= 1) {
-    if ((int)threadIdx.x < off) sh[threadIdx.x] += sh[threadIdx.x + off];
-    __syncthreads();
+void ew_cells_make(const double* box, double rcut, int n, EwCells* c) {
+  // about four cells per particle at most, so that a sparse box does not
+  // spend its time on empty cells
+  const int cap = std::max(2, std::min(64, (int)std::cbrt(4.0 * n)));
+  c->ncell = 1;
+  for (int a = 0; a < 3; a++) {
+    const int split = a == 0 ? 4 : 2, top = a == 0 ? 2 * cap : cap;
+    c->box[a] = box[a];
+    c->len[a] = (float)(box[a] / rcut);
+    // the margin keeps rounding from letting a pair within rcut lie one cell
+    // beyond the reach
+    const double fit = box[a] / rcut * split * (1.0 - 1e-9);
+    c->nc[a] = fit >= top ? top : std::max(1, (int)fit);
+    const double need = rcut / box[a] * c->nc[a] * (1.0 + 1e-12);
+    c->reach[a] = need >= c->nc[a] ? c->nc[a] : (int)std::ceil(need);
+    c->ncell *= c->nc[a];
   }
-  if (threadIdx.x == 0) energy[0] = sh[0] + self2[0];
 }
 
-hipError_t launch_ew_cells(const void* xyzq, int n, const EwCells& c, int* cell_of, int* counts,
-                           int* starts, int* fill, int* tmp, int* sidx, void* sx,
-                           hipStream_t s) {
+void ew_filter_make(const EwCells& c, EwPair* p) {
+  // Positions in units of rcut are rounded to 24 bits, shifted and
+  // subtracted, cell edges multiplied out: each is off by less than 8 * 2^-24
+  // of the longest edge, the squares by a few units in the last place.
+  const double len = std::max(1.0, (double)std::max(c.len[0], std::max(c.len[1], c.len[2])));
+  const double slack = 16.0 * len / 16777216.0;
+  p->slack = (float)slack;
+  p->filter2 = (float)((1.0 + slack) * (1.0 + slack) * (1.0 + 1e-6));
+}
+
+hipError_t launch_ew_cells(const void* xyzq, int n, const EwCells& c, double rcut, int* cell_of,
+                           int* rank, int* counts, int* starts, int* tmp, int* sidx, void* sx,
+                           void* sf, double* q2, hipStream_t s) {
   k_zero_i32<<<blocks_for(c.ncell, 256, 1024), 256, 0, s>>>(counts, c.ncell);
+  const unsigned g = blocks_for(n > 0 ? n : 1, 256, 4096);
+  k_ew_cell_count<<<kEwCountBlocks, 256, 0, s>>>((const P4<double>*)xyzq, n, c, cell_of, rank,
+                                                 counts, q2);
+  k_ew_scan<<<1, 1024, 0, s>>>(counts, c.ncell, starts);
   if (n > 0) {
-    const unsigned g = blocks_for(n, 256, 4096);
-    k_ew_cell_count<<<g, 256, 0, s>>>((const P4<double>*)xyzq, n, c, cell_of, counts);
-  }
-  k_ew_scan<<<1, 1024, 0, s>>>(counts, c.ncell, starts, fill);
-  if (n > 0) {
-    const unsigned g = blocks_for(n, 256, 4096);
-    k_ew_scatter<<<g, 256, 0, s>>>(n, cell_of, starts, fill, tmp);
-    k_ew_sort<<<g, 256, 0, s>>>(n, cell_of, starts, counts, tmp, (const P4<double>*)xyzq, sidx,
-                                (P4<double>*)sx);
+    k_ew_scatter<<<g, 256, 0, s>>>(n, cell_of, rank, starts, tmp);
+    k_ew_sort<<<g, 256, 0, s>>>(n, c, 1.0 / rcut, cell_of, starts, tmp, (const P4<double>*)xyzq,
+                                sidx, (P4<double>*)sx, (P4<float>*)sf);
   }
   return hipGetLastError();
 }
 
-hipError_t launch_ew_force(const EwCells& c, const EwPair& p, const int* starts,
-                           const int* counts, const int* sidx, const void* sx, const int* xofs,
-                           const int* xlist, double* gx, double* gy, double* gz,
+hipError_t launch_ew_force(int n, const EwCells& c, const EwPair& p, const int* starts,
+                           const int* sidx, const void* sx, const void* sf, const int* xofs,
+                           const int* xlist, const double* erfcx, double* gx, double* gy, double* gz,
                            double* partials, hipStream_t s) {
-  k_ew_force<<<c.ncell, kEwThreads, 0, s>>>(c, p, starts, counts, sidx, (const P4<double>*)sx,
-                                            xofs, xlist, gx, gy, gz, partials);
+  if (n <= 0) return hipSuccess;
+  const unsigned g = (unsigned)((n + kEwWaves - 1) / kEwWaves);
+  const P4<double>* x = (const P4<double>*)sx;
+  const P4<float>* f = (const P4<float>*)sf;
+  // no axis is short enough to visit all its cells: every image is a shift
+  const bool fold = c.nc[0] <= 2 * c.reach[0] + 2 || c.nc[1] <= 2 * c.reach[1] + 1 ||
+                    c.nc[2] <= 2 * c.reach[2] + 1;
+  if (fold)
+    k_ew_force<true><<<g, 64 * kEwWaves, 0, s>>>(n, c, p, starts, sidx, x, f, xofs, xlist, erfcx,
+                                                 gx, gy, gz, partials);
+  else
+    k_ew_force<false><<<g, 64 * kEwWaves, 0, s>>>(n, c, p, starts, sidx, x, f, xofs, xlist,
+                                                  erfcx, gx, gy, gz, partials);
   return hipGetLastError();
 }
 
-hipError_t launch_ew_finalize(const double* partials, int ncell, const double* self2,
+hipError_t launch_ew_finalize(const double* partials, int n, const double* q2, double self,
                               double* energy, hipStream_t s) {
-  k_ew_finalize<<<1, 256, 0, s>>>(partials, ncell, self2, energy);
+  k_ew_finalize<<<1, 1024, 0, s>>>(partials, n, q2, kEwCountBlocks, self, energy);
   return hipGetLastError();
 }
 

@@ -456,23 +456,39 @@ hipError_t launch_pme_gather(bool ct_dbl, bool at_dbl, int order, const void* xy
 
 // ---- Ewald direct space (ewald_pme.hip) ----------------------------------
 struct EwCells {
-  int nc[3];      // cells per axis (1 when fewer than 3 cells of edge >= rcut fit)
+  int nc[3];      // cells per axis
+  int reach[3];   // cells on either side that a pair within rcut can span
   int ncell;
   double box[3];
+  float len[3];   // box edges in units of rcut
 };
 struct EwPair {
   double rcut2, ccelec, inv_sqrt2sigma, inv_2sigmasq, two_sqrtpi;
+  // 32-bit filter in units of rcut: bound on r2 of a pair within rcut, and
+  // on the rounding of positions and cell edges
+  float filter2, slack;
 };
-// cell lists: counts/starts/fill [ncell], cell_of/tmp/sidx [n], sx [n] double4
-hipError_t launch_ew_cells(const void* xyzq, int n, const EwCells& c, int* cell_of, int* counts,
-                           int* starts, int* fill, int* tmp, int* sidx, void* sx,
-                           hipStream_t s);
-// xofs/xlist: symmetric exclusion lists (CSR over particles; xofs NULL: none)
-hipError_t launch_ew_force(const EwCells& c, const EwPair& p, const int* starts,
-                           const int* counts, const int* sidx, const void* sx, const int* xofs,
-                           const int* xlist, double* gx, double* gy, double* gz,
-                           double* partials, hipStream_t s);
-hipError_t launch_ew_finalize(const double* partials, int ncell, const double* self2,
+constexpr int kEwCountBlocks = 256;
+// cells of n particles: rcut/4 along x, rcut/2 along y and z, at most about
+// four per particle
+void ew_cells_make(const double* box, double rcut, int n, EwCells* c);
+void ew_filter_make(const EwCells& c, EwPair* p);
+// cell lists: counts [ncell], starts [ncell + 1], cell_of/rank/tmp/sidx [n],
+// sx [n] double4, sf [n] float4; q2 [kEwCountBlocks] partial sums of q^2
+hipError_t launch_ew_cells(const void* xyzq, int n, const EwCells& c, double rcut, int* cell_of,
+                           int* rank, int* counts, int* starts, int* tmp, int* sidx, void* sx,
+                           void* sf, double* q2, hipStream_t s);
+// host table of erfcx that launch_ew_force reads from device memory
+const double* ew_erfcx_table();
+size_t ew_erfcx_bytes();
+// xofs/xlist: symmetric exclusion lists (CSR over particles; xofs NULL: none);
+// erfcx: device copy of ew_erfcx_table; partials [n] energies
+hipError_t launch_ew_force(int n, const EwCells& c, const EwPair& p, const int* starts,
+                           const int* sidx, const void* sx, const void* sf, const int* xofs,
+                           const int* xlist, const double* erfcx, double* gx, double* gy,
+                           double* gz, double* partials, hipStream_t s);
+// energy = sum of the partials + self * sum of q^2
+hipError_t launch_ew_finalize(const double* partials, int n, const double* q2, double self,
                               double* energy, hipStream_t s);
 
 // ---- Ewald reciprocal sum (ewald_pme.hip) --------------------------------

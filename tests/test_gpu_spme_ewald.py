@@ -163,6 +163,53 @@ def test_ewald_direct_fp64(case):
     assert eg2 == eg and torch.equal(f2, f)
 
 
+# box edges in units of rcut around the places where the cell walk changes:
+# one cell, all cells of an axis visited, every image a shift; x cells are
+# rcut/4, y and z cells rcut/2
+EW_EDGES = [((0.7, 0.7, 0.7), 2, 1.0), ((0.7, 1.6, 3.3), 65, 1.0), ((2.4, 2.4, 2.4), 200, 1.0),
+            ((2.51, 2.99, 3.0), 200, 1.0), ((3.2, 2.4, 3.1), 129, 1.0), ((5.0, 0.9, 2.5), 257, 1.0),
+            ((40.0, 3.0, 3.0), 64, 1.0), ((4.0, 4.0, 4.0), 1, 1.0),
+            # erfc far out: rcut / (sqrt(2) sigma) = 8.8 and 35
+            ((3.0, 3.5, 4.0), 300, 0.08), ((3.0, 3.0, 3.0), 150, 0.02)]
+
+
+@pytest.mark.parametrize("edges,n,width", EW_EDGES)
+def test_ewald_direct_cell_edges(edges, n, width):
+    """The direct sum where the candidate ranges change form, against the
+    oracle: coordinates on box faces and several boxes outside, six
+    exclusions per atom, and Gaussian widths down to rcut/50.  A pair term is
+    a dozen FP64 roundings and the sums run over at most n terms, so a
+    component is off by less than (12 + n) 2^-53 of the sum of its terms'
+    magnitudes, bounded here by n times the largest pair force."""
+    rcut = 6.0
+    box = tuple(rcut * e for e in edges)
+    rng = np.random.default_rng(n)
+    x = systems.random_alternating(n, 1.0, seed=n) * np.array([*box, 1.0])
+    x[:, :3] += rng.integers(-3, 4, size=(n, 3)) * np.array(box)
+    x[0, :3] = 0.0
+    x[-1, :3] = box
+    if n == 2:  # both records at one point otherwise
+        x[-1, :3] = np.array(box) * 0.4
+    elif n > 2:
+        x[1, :3] = (box[0], 0.5 * box[1], 0.0)
+        x[-1, :3] = (0.5 * box[0], box[1], 0.25 * box[2])
+    ib, nb = [], []
+    for j in range(n):
+        nb.extend(i + 1 for i in range(j + 1, min(j + 4, n)))
+        ib.append(len(nb))
+    sigma = width * rcut / 2.0
+    e, g = orc.ewald_direct(sigma, rcut, box, x, ib, nb)
+    d = api.CpuEwaldDirect(sigma, rcut, *box)
+    d.setupExclusions(n, ib, nb)
+    f = torch.zeros((3, n), dtype=F64, device="cuda")
+    eg = d.calcForceEnergy(n, dev(x), f[0], f[1], f[2])
+    fg = host(f).T
+    scale = max(np.max(np.abs(g)), 1e-300)
+    print(f"E {e:.12e} gpu {eg:.12e} max dF/F {np.max(np.abs(fg - g)) / scale:.1e}", flush=True)
+    assert np.max(np.abs(fg - g)) <= (12 + n) * n * 2.0 ** -53 * scale
+    assert abs(eg - e) <= (12 + n) * 2.0 ** -53 * n * max(abs(e), 332.0716 / sigma)
+
+
 def test_total_electrostatics_like_test48k():
     """cpu_gse.cpp:332-389 adds the direct-space sum to each reciprocal method
     and compares with Ewald.  On the 3k water box, GSE-k (this library) plus

@@ -245,7 +245,7 @@ struct Engine {
     bin.bshift = nullptr;
     if (brick_flush) {
       const size_t vol = (size_t)shape.Lx * shape.Ly * shape.Lz;
-      GSECHK(bricks.ensure((acc32() ? 4 : 8) * vol * (size_t)shape.nbins));
+      GSECHK(bricks.ensure((acc32() ? 4 : 8) * vol * (size_t)shape.nbins + kBrickPad));
       GSECHK(bshift.ensure(sizeof(int) * (size_t)shape.nbins));
       bin.bricks = bricks.p;
       bin.bshift = bshift.as<int>();
@@ -1156,6 +1156,7 @@ gse_status_t gse_gauss_charge_spread_charge_to_grid_noalloc(gse_gauss_charge_t h
                o_perm = take(sizeof(int) * slots), o_loc = take(sizeof(int) * slots),
                o_sorted = take(4 * tsize(dbl) * slots), o_g64 = take(8 * npts),
                o_bricks = flush ? take((acc32 ? 4 : 8) * (size_t)b.Lx * b.Ly * b.Lz * nb) : 0,
+               // at least kBrickPad bytes after the bricks
                o_bshift = flush ? take(sizeof(int) * (size_t)nb) : 0;
   if (off > kNoAllocScratchBytes)
     return fail(GSE_ERROR_INVALID_VALUE,

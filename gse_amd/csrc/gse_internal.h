@@ -180,6 +180,9 @@ hipError_t launch_fixed_to_grid(bool ct_double, const unsigned long long* grid64
                                 void* out, size_t count, const Binning& w,
                                 bool clear, hipStream_t s);
 
+// readable bytes after the last brick: a 16-byte load may start at its last
+// element
+constexpr size_t kBrickPad = 16;
 // Brick-store flush: usable for this shape (LDS path, bounded brick overlap)?
 bool brick_reduce_ok(const Geom& g, const BinShape& b);
 bool spread_mma_ok(bool dbl, const Geom& g, const BinShape& b, bool normalize, bool acc32,
@@ -187,7 +190,7 @@ bool spread_mma_ok(bool dbl, const Geom& g, const BinShape& b, bool normalize, b
 // Which kernel converts a spread's fixed-point sums into the grid:
 enum ReducePath : int {
   kReduceAtomic = 0,   // bricks added with 64-bit atomics, then k_fixed_to_grid
-  kReduceGeneric = 1,  // k_brick_reduce, one thread per grid point
+  kReduceGeneric = 1,  // k_brick_reduce, any bin shape and grid size
   kReduceTile4 = 2,    // k_brick_reduce_tile4 (32-bit bricks, 16-byte pieces)
   kReduceTile4NT = 3,  // the same with non-temporal brick loads
   kReduceTile2 = 4,    // k_brick_reduce_tile2 (64-bit bricks, two x points per thread)

@@ -698,6 +698,45 @@ def test_reduce_tile2_gives_identical_grids(dt, lds32):
         api.set_tuning(reduce_tile2=keys["reduce_tile2"], spread_lds32=keys["spread_lds32"])
 
 
+# grid sizes around multiples of the bin edge (last bins of 1 to 8 cells),
+# spacings with 7- and 9-cell supports (4-cell bins), bricks that wrap onto
+# themselves, one bin per axis
+REDUCE_SHAPES = [((54, 63, 50), 0.99), ((57, 33, 41), 1.0), ((26, 47, 31), 0.9),
+                 ((20, 20, 20), 1.0), ((17, 9, 28), 1.0), ((25, 24, 36), 0.7), ((8, 30, 12), 1.1)]
+
+
+@pytest.mark.parametrize("dt,lds32", [(F32, 1), (F64, 1), (F32, 0)],
+                         ids=["F32", "F64", "F32-int64"])
+@pytest.mark.parametrize("dims,h", REDUCE_SHAPES)
+def test_brick_reduce_any_shape(dims, h, dt, lds32):
+    """The brick reduce of grids that are not whole 8^3 bins against adding
+    the bricks with 64-bit atomics: the same integers, so the same bits, with
+    a cluster that overfills its bin."""
+    rng = np.random.default_rng(sum(dims))
+    box = tuple(h * m for m in dims)
+    n = 900
+    xyzq = np.empty((n, 4))
+    xyzq[:, :3] = rng.random((n, 3)) * box
+    xyzq[: n // 2, :3] = np.array(box) - 0.4 * h + rng.random((n // 2, 3)) * 0.3 * h
+    xyzq[:, 3] = rng.standard_normal(n)
+    p = orc.Params(dims, box, 2.12)
+    keys = api.get_tuning()
+    try:
+        api.set_tuning(spread_lds32=lds32)
+        outs = []
+        for flush, path in ((1, "generic"), (0, "atomic")):
+            api.set_tuning(spread_flush=flush)
+            g = api.CpuGaussCharge(dt, dt, *dims)
+            rho = grid(dims, dt)
+            g.spreadChargeToGrid(p.sigma1, p.rcut1, n, to_dev(xyzq, dt), *box, rho)
+            if not g.layout()["direct"]:
+                assert g.layout()["reduce"] in (path, "atomic")
+            outs.append(rho)
+        assert torch.equal(outs[0], outs[1])
+    finally:
+        api.set_tuning(spread_flush=keys["spread_flush"], spread_lds32=keys["spread_lds32"])
+
+
 def test_numcoord_beyond_xyzq_is_rejected():
     """numCoord larger than the particle tensor is refused on the host, before
     any kernel could read past the allocation."""

@@ -819,18 +819,21 @@ struct gse_gser_s {
   DevBuf rho;
 };
 
-// GSE-u (CpuGSEu.h): the core's rhoS is the sigma1 grid; N convolved terms
+// GSE-u (CpuGSEu.h): the core's rhoS is the sigma1 grid; N convolved terms,
+// taken kUTerms at a time from the widest down
 struct gse_gseu_s {
   gse_gsek_s* core = nullptr;
   int N = 0;
   double b = 0.0;
-  std::vector<double> sig, fac;        // sigma_j and (2 pi sigma_j^2)^(3/2)/sigma_j
-  struct Taps3 {
-    DevBuf t[3];
-    int R[3];
+  struct Chunk {
+    UTaps t[2];          // y and z taps of the chunk's terms
+    size_t xtap = 0;     // first of its x taps in `taps`
+    int Rx = 0;
+    size_t at[2][kUTerms] = {};  // first y and z tap of each term in `taps`
   };
-  std::vector<Taps3*> taps;            // the three tap arrays and radii of each term
-  std::vector<DevBuf*> terms;          // rhoG_j
+  std::vector<Chunk> chunks;
+  DevBuf taps;           // every tap, FP64
+  DevBuf a, b2;          // the terms of a chunk after the x and after the y pass
 };
 
 // Ewald direct space + self energy (CpuEwaldDirect.h:10-44)
@@ -844,6 +847,66 @@ struct gse_ewald_direct_s {
 };
 
 namespace {
+
+// Terms of a GSE-u handle (CpuGSEu.cpp:51-66): sigma_j = sqrt(sigma^2 b^(2j) -
+// 2 sigma1^2), radius ceil(rcut_j / h), the on-grid taps of
+// CpuGaussCharge.cpp:406-433 and the factor (2 pi sigma_j^2)^(3/2) / sigma_j,
+// widest first, in chunks of kUTerms.
+gse_status_t gseu_terms(gse_gseu_s* h, double sigma, double ls1) {
+  const gse_gsek_s* c = h->core;
+  const double hh[3] = {c->bx / c->X, c->by / c->Y, c->bz / c->Z};
+  std::vector<double> all;
+  for (int top = h->N - 1; top >= 0; top -= kUTerms) {
+    const int nt = std::min(kUTerms, top + 1);
+    std::vector<double> tap[kUTerms][3];
+    int R[kUTerms][3];
+    for (int k = 0; k < nt; k++) {
+      const int j = top - k;
+      const double s2 = sigma * sigma * std::pow(h->b, 2 * j) - 2 * c->sigma1 * c->sigma1;
+      const double sj = std::sqrt(s2);
+      if (!(sj > 0) || !std::isfinite(sj))
+        return fail(GSE_ERROR_INVALID_VALUE, "sigma_%d is not positive", j);
+      const double rc = ls1 * std::sqrt(2.0) * sj, inv_2sigmasq = 1.0 / (2.0 * sj * sj);
+      const double pref = std::pow(2.0 * M_PI * sj * sj, -1.5) * hh[0] * hh[1] * hh[2] *
+                          (std::pow(2 * M_PI * sj * sj, 3.0 / 2.0) / std::pow(sj * sj, 1.0 / 2.0));
+      for (int a = 0; a < 3; a++) {
+        R[k][a] = (int)std::ceil(rc / hh[a]);
+        for (int ii = -R[k][a]; ii <= R[k][a]; ii++)
+          tap[k][a].push_back((a == 2 ? pref : 1.0) *
+                              std::exp(-hh[a] * hh[a] * (double)(ii * ii) * inv_2sigmasq));
+      }
+    }
+    gse_gseu_s::Chunk ch;
+    for (int k = 0; k < nt; k++) ch.Rx = std::max(ch.Rx, R[k][0]);
+    ch.xtap = all.size();
+    all.resize(ch.xtap + (size_t)(2 * ch.Rx + 1) * kUTerms, 0.0);
+    for (int k = 0; k < nt; k++)
+      for (int i = 0; i < (int)tap[k][0].size(); i++)
+        all[ch.xtap + (size_t)(i + ch.Rx - R[k][0]) * kUTerms + k] = tap[k][0][i];
+    for (int a = 1; a < 3; a++) {
+      UTaps& t = ch.t[a - 1];
+      t = UTaps{};
+      t.nterm = nt;
+      for (int k = 0; k < nt; k++) {
+        t.R[k] = R[k][a];
+        const size_t at = all.size() + kUTile - 1;
+        all.resize(at + 2 * R[k][a] + 2 * kUTile, 0.0);
+        std::copy(tap[k][a].begin(), tap[k][a].end(), all.begin() + at);
+        ch.at[a - 1][k] = at;
+      }
+    }
+    h->chunks.push_back(ch);
+  }
+  GSECHK(h->taps.ensure(sizeof(double) * all.size()));
+  HIPCHK(hipMemcpy(h->taps.p, all.data(), sizeof(double) * all.size(), hipMemcpyHostToDevice));
+  for (auto& ch : h->chunks)
+    for (int a = 0; a < 2; a++)
+      for (int k = 0; k < ch.t[a].nterm; k++) ch.t[a].tap[k] = h->taps.as<double>() + ch.at[a][k];
+  const size_t gb = tsize(c->ct_dbl) * (size_t)c->X * c->Y * c->Z * std::min(h->N, kUTerms);
+  GSECHK(h->a.ensure(gb));
+  GSECHK(h->b2.ensure(gb));
+  return GSE_SUCCESS;
+}
 
 // separable sigma taps of spreadChargeOnGrid (CpuGaussCharge.cpp:406-433)
 gse_status_t make_ongrid_taps(bool dbl, int X, int Y, int Z, double sigma, double rcut,
@@ -2287,26 +2350,7 @@ gse_status_t gse_gseu_create(gse_gseu_t* out, gse_dtype_t at, gse_dtype_t ct, in
   h->core = core;
   h->N = N;
   h->b = b;
-  gse_status_t st = GSE_SUCCESS;
-  const size_t gb = tsize(core->ct_dbl) * (size_t)X * Y * Z;
-  for (int j = 0; j < N && st == GSE_SUCCESS; j++) {
-    // CpuGSEu.cpp:52-56
-    const double sj = std::sqrt(sigma * sigma * std::pow(b, 2 * j) -
-                                2 * core->sigma1 * core->sigma1);
-    if (!(sj > 0) || !std::isfinite(sj)) {
-      st = fail(GSE_ERROR_INVALID_VALUE, "sigma_%d is not positive", j);
-      break;
-    }
-    h->sig.push_back(sj);
-    h->fac.push_back(std::pow(2 * M_PI * sj * sj, 3.0 / 2.0) / std::pow(sj * sj, 1.0 / 2.0));
-    auto* t3 = new gse_gseu_s::Taps3();
-    h->taps.push_back(t3);
-    st = make_ongrid_taps(core->ct_dbl, X, Y, Z, sj, ls1 * std::sqrt(2.0) * sj, bx, by, bz, t3->t,
-                          t3->R);
-    DevBuf* g = new DevBuf();
-    h->terms.push_back(g);
-    if (st == GSE_SUCCESS) st = g->ensure(gb);
-  }
+  const gse_status_t st = gseu_terms(h, sigma, ls1);
   if (st != GSE_SUCCESS) {
     gse_gseu_destroy(h);
     return st;
@@ -2318,14 +2362,7 @@ gse_status_t gse_gseu_create(gse_gseu_t* out, gse_dtype_t at, gse_dtype_t ct, in
 gse_status_t gse_gseu_destroy(gse_gseu_t h) {
   if (!h) return GSE_SUCCESS;
   gse_gsek_destroy(h->core);
-  for (auto* t3 : h->taps) {
-    for (int a = 0; a < 3; a++) t3->t[a].release();
-    delete t3;
-  }
-  for (DevBuf* g : h->terms) {
-    g->release();
-    delete g;
-  }
+  for (DevBuf* g : {&h->taps, &h->a, &h->b2}) g->release();
   delete h;
   return GSE_SUCCESS;
 }
@@ -2343,17 +2380,13 @@ gse_status_t gse_gseu_spread_charge1(gse_gseu_t h, int n, const void* xyzq) {
 gse_status_t gse_gseu_solve_poisson(gse_gseu_t h) {
   if (!h) return fail(GSE_ERROR_INVALID_VALUE, "handle is NULL");
   gse_gsek_s* c = h->core;
-  const size_t np = (size_t)c->X * c->Y * c->Z;
-  for (int j = 0; j < h->N; j++) {
-    GSECHK(conv3(c->ct_dbl, c->X, c->Y, c->Z, h->taps[j]->R, h->taps[j]->t, c->rhoS.p,
-                 h->terms[j]->p, c->tmp, c->tmp2, c->stream));
-    HIPCHK(launch_grid_scale(c->ct_dbl, h->terms[j]->p, h->terms[j]->p, np, h->fac[j], c->stream));
+  // phiM = rhoG_{N-1} + ... + rhoG_0 (CpuGSEu.cpp:60-66)
+  bool add = false;
+  for (const auto& k : h->chunks) {
+    HIPCHK(launch_useries(c->ct_dbl, c->X, c->Y, c->Z, k.t, h->taps.as<double>() + k.xtap, k.Rx,
+                          c->rhoS.p, h->a.p, h->b2.p, c->phiM.p, add, c->stream));
+    add = true;
   }
-  // phiM = rhoG_{N-1} + ... + rhoG_0, added in that order (CpuGSEu.cpp:60-66)
-  HIPCHK(hipMemcpyAsync(c->phiM.p, h->terms[h->N - 1]->p, tsize(c->ct_dbl) * np,
-                        hipMemcpyDeviceToDevice, c->stream));
-  for (int j = h->N - 2; j >= 0; j--)
-    HIPCHK(launch_grid_add(c->ct_dbl, c->phiM.p, h->terms[j]->p, np, c->stream));
   return GSE_SUCCESS;
 }
 

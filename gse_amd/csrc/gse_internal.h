@@ -412,10 +412,6 @@ hipError_t launch_add_sym6(const double* partials, int nblocks, double* vir9, hi
 hipError_t launch_corrections_finalize(const double* partials, int nblocks, double sigma,
                                        double bx, double by, double bz, double ccelec,
                                        double* out, hipStream_t s);
-// out[i] = f * in[i] (out may be in); out[i] += in[i]
-hipError_t launch_grid_scale(bool dbl, void* out, const void* in, size_t n, double f,
-                             hipStream_t s);
-hipError_t launch_grid_add(bool dbl, void* out, const void* in, size_t n, hipStream_t s);
 // sums n per-particle values of `ncomp` components laid out [ncomp][n]
 hipError_t launch_sum_columns(const double* v, int n, int ncomp, double* partials,
                               hipStream_t s);
@@ -431,6 +427,21 @@ hipError_t launch_efield(bool dbl, int X, int Y, int Z, double bx, double by,
 hipError_t launch_conv_pass(bool dbl, int pass, int X, int Y, int Z, int R,
                             const void* taps, const void* in, void* out,
                             hipStream_t s, bool sym = false);
+
+// u-series potential: phi (+)= sum over up to kUTerms terms of the separable
+// Gaussians rho * x * y * z, sums in FP64.  taps[0] / taps[1]: y / z taps
+// (device, tap[k][-(kUTile-1) .. 2R + 2 kUTile) with zeros outside [0, 2R],
+// the terms' factors in the z taps); xtap: [2Rx+1][kUTerms], zeros where a
+// term is narrower; a, b: kUTerms grids each.
+constexpr int kUTerms = 4, kUTile = 4;
+struct UTaps {
+  int nterm;
+  int R[kUTerms];
+  const double* tap[kUTerms];
+};
+hipError_t launch_useries(bool dbl, int X, int Y, int Z, const UTaps* taps, const double* xtap,
+                          int Rx, const void* rho, void* a, void* b, void* phi, bool add,
+                          hipStream_t s);
 
 // charge statistics for the closed-form corrections: out[0] = sum q,
 // out[1] = sum q^2 (FP64 partials -> finalize)

@@ -105,6 +105,25 @@ def test_gseu_fp64(case, N, b):
     assert rel(host(o["force"]).T, f) <= TOL
 
 
+@pytest.mark.parametrize("N,b,dims,h", [
+    (1, 1.168, (17, 15, 13), 1.0), (4, 1.168, (37, 50, 21), 1.1), (5, 1.168, (18, 35, 27), 0.8),
+    (6, 1.3, (9, 33, 20), 1.0)], ids=["one", "chunk", "chunk+1", "wide"])
+def test_gseu_chunks_and_ragged_grids(N, b, dims, h):
+    """One term, a full chunk of terms and one more, on grids that are no
+    multiple of the column tiles, with radii up to several grid lengths."""
+    box = tuple(h * m for m in dims)
+    x = systems.water_box(60, 1.0, seed=N, wrap=False)
+    x[:, :3] *= np.array(box)
+    p = orc.Params(dims, box, 2.12)
+    e, f, phi = orc.gseu_step(p, N, b, x)
+    g = api.CpuGSEu(F64, F64, N, b, *dims, 2.12, 0.4, 3.0, 3.0, *box)
+    for _ in range(2):  # the second step starts from the first one's potential
+        o = g.step(dev(x), force=True)
+        assert abs(float(host(o["energy"])[0]) - e) <= TOL * abs(e)
+        assert rel(host(o["force"]).T, f) <= TOL
+        assert rel(host(g.getPhi()), phi) <= TOL
+
+
 def test_gseu_gser_fp32_water():
     xyzq, L, M, s = systems.make("water_3k_M32")
     x32 = dev(xyzq, F32)

@@ -800,7 +800,9 @@ struct gse_pme_recip_s {
   double recip3[3] = {0, 0, 0};  // of the last spread (gather and scalar_sum reuse it)
   int n_last = 0;
   KSolverFFTOnly* fft = nullptr;
-  DevBuf grid64, grid, spec, prefac, partials, stats, tmp2;
+  DevBuf grid64, grid, spec, prefac, partials, stats, tmp2, counts, ovf, sorted, bricks, bshift;
+  int cur = 0;         // the statistics buffer of the next spread
+  bool clean = false;  // counts and that buffer are zero
   hipStream_t stream = nullptr;
 };
 
@@ -1845,15 +1847,6 @@ gse_status_t pme_recip3(const double* recip, double* r3) {
 }
 
 // the int64 -> grid conversion reads max |q| and the count from a Binning
-Binning pme_binning(gse_pme_recip_s* h, int n) {
-  Binning w;
-  w.n = n;
-  w.stats = h->stats.as<BinStats>();
-  w.images = 1;
-  w.pref_bound = 1.0;
-  return w;
-}
-
 constexpr double kPmeCcelec = 332.0716;  // CudaPMERecip.h:25
 
 }  // namespace
@@ -1886,7 +1879,7 @@ gse_status_t gse_pme_recip_create(gse_pme_recip_t* out, gse_dtype_t at, gse_dtyp
   if (st == GSE_SUCCESS) st = h->spec.ensure(2 * tsize(h->ct_dbl) * nk);
   if (st == GSE_SUCCESS) st = h->prefac.ensure(sizeof(double) * (size_t)(nfftx + nffty + nfftz));
   if (st == GSE_SUCCESS) st = h->partials.ensure(sizeof(double) * 7 * kPmeSumBlocks);
-  if (st == GSE_SUCCESS) st = h->stats.ensure(sizeof(BinStats));
+  if (st == GSE_SUCCESS) st = h->stats.ensure(2 * sizeof(BinStats));
   if (st == GSE_SUCCESS) st = h->tmp2.ensure(sizeof(double) * (kRedBlocks * 2 + 2));
   if (st == GSE_SUCCESS) {
     std::vector<double> pf((size_t)nfftx + nffty + nfftz);
@@ -1913,7 +1906,8 @@ gse_status_t gse_pme_recip_destroy(gse_pme_recip_t h) {
     h->fft->fft.release();
     delete h->fft;
   }
-  for (DevBuf* b : {&h->grid64, &h->grid, &h->spec, &h->prefac, &h->partials, &h->stats, &h->tmp2})
+  for (DevBuf* b : {&h->grid64, &h->grid, &h->spec, &h->prefac, &h->partials, &h->stats, &h->tmp2,
+                    &h->counts, &h->ovf, &h->sorted, &h->bricks, &h->bshift})
     b->release();
   delete h;
   return GSE_SUCCESS;
@@ -1934,12 +1928,35 @@ gse_status_t gse_pme_recip_spread_charge(gse_pme_recip_t h, const void* xyzq, in
   std::memcpy(h->recip3, r3, sizeof(r3));
   h->n_last = ncoord;
   hipStream_t s = h->stream;
-  HIPCHK(launch_pme_qmax(h->ct_dbl, xyzq, ncoord, r3, h->stats.as<BinStats>(), s));
-  HIPCHK(launch_pme_spread(h->ct_dbl, h->order, xyzq, ncoord, h->X, h->Y, h->Z, r3,
-                           h->stats.as<BinStats>(), h->grid64.as<unsigned long long>(), s));
-  const Binning w = pme_binning(h, ncoord);
-  HIPCHK(launch_fixed_to_grid(h->ct_dbl, h->grid64.as<unsigned long long>(), h->grid.p,
-                              (size_t)h->X * h->Y * h->Z, w, true, s));
+  const PmeGrid a = pme_grid_make(h->X, h->Y, h->Z, h->order, r3);
+  // twice the mean occupancy plus a margin; the rest spreads by itself
+  const int nb = a.b.nbins, cap = (int)((2LL * ncoord / nb + 32 + 15) / 16 * 16);
+  const size_t vol = (size_t)a.b.Lx * a.b.Ly * a.b.Lz;
+  GSECHK(h->counts.ensure(sizeof(int) * (size_t)nb));
+  GSECHK(h->bshift.ensure(sizeof(int) * (size_t)nb));
+  GSECHK(h->bricks.ensure(8 * vol * nb + kBrickPad));
+  GSECHK(h->sorted.ensure(4 * tsize(h->ct_dbl) * (size_t)nb * cap));
+  GSECHK(h->ovf.ensure(sizeof(int) * (size_t)std::max(ncoord, 1)));
+  BinStats* st = h->stats.as<BinStats>() + h->cur;
+  if (!h->clean) HIPCHK(launch_bin_clear(h->counts.as<int>(), nb, st, s));
+  h->clean = false;
+  HIPCHK(launch_pme_bin(h->ct_dbl, xyzq, ncoord, a, cap, h->counts.as<int>(), st,
+                        h->ovf.as<int>(), h->sorted.p, s));
+  HIPCHK(launch_pme_spread(h->ct_dbl, h->order, xyzq, ncoord, a, cap, h->counts.as<int>(), st,
+                           h->stats.as<BinStats>() + (h->cur ^ 1), h->ovf.as<int>(), h->sorted.p,
+                           h->bricks.p, h->bshift.as<int>(), h->grid64.as<unsigned long long>(),
+                           s));
+  Binning w;
+  w.n = ncoord;
+  w.stats = st;
+  w.pref_bound = 1.0;
+  w.bricks = h->bricks.p;
+  w.bshift = h->bshift.as<int>();
+  const Geom g = make_geom(h->X, h->Y, h->Z, 1.0, 1.0, 1.0, 1.0);
+  HIPCHK(launch_brick_reduce_list(h->ct_dbl, false, g, a.b, w, h->grid64.as<unsigned long long>(),
+                                  h->grid.p, s));
+  h->cur ^= 1;
+  h->clean = true;
   return GSE_SUCCESS;
 }
 

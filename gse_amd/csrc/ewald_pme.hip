@@ -1,12 +1,13 @@
 // Comparators beside the GSE path, on the same device infrastructure:
 //
 // SPME reciprocal space (the reference's cuda/CudaPMERecip.cu, order 4/6/8):
-//   k_pme_qmax      max |q| and the rejected-particle count of one call
-//   k_pme_spread    B-spline charge spread into the int64 fixed-point grid
-//                   (one lane per (x, y) spline offset, a loop over z; the
-//                   same exponent rule as the GSE spread, so the grid is
-//                   bit-identical for any particle order); the conversion to
-//                   the compute type is the GSE path's k_fixed_to_grid
+//   k_pme_bin       particles into bins of 8^3 cells, max |q| and the
+//                   rejected-particle count of one call
+//   k_pme_spread    B-spline spread of one bin into an int64 fixed-point
+//                   brick in LDS (one lane per (x, y) spline offset, a loop
+//                   over z; the same exponent rule as the GSE spread, so the
+//                   grid is bit-identical for any particle order); the GSE
+//                   path's k_brick_reduce sums and converts the bricks
 //   k_pme_scalar_sum  the spectrum times the SPME kernel with FP64 energy and
 //                   virial partial sums per workgroup (fixed order)
 //   k_pme_finalize  energy and the 3x3 virial from the partial sums
@@ -20,11 +21,11 @@
 //   k_ew_cell_count / k_ew_scan / k_ew_scatter / k_ew_sort
 //                   particles into cells, each cell's list in ascending
 //                   particle index (deterministic order); partial sums of q^2
-//   k_ew_force      one wave per group of particles: candidates of the cells
+//   k_ew_force      one wave per particle: candidates of the cells
 //                   within reach pass a 32-bit distance filter into a queue,
 //                   full queues are evaluated in FP64 with the reference's
 //                   operand order and minimum-image loops
-//   k_ew_finalize   energy of the groups and the self term
+//   k_ew_finalize   energy of the particles and the self term
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -40,13 +41,6 @@ template <typename T>
 struct alignas(4 * sizeof(T)) P4 {
   T x, y, z, w;
 };
-
-__global__ void k_clear_stats(BinStats* st) {
-  st->qmax_bits = 0ull;
-  st->invalid = 0;
-  st->overflow = 0;
-  st->spill = 0;
-}
 
 __global__ void k_zero_i32(int* p, int n) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0;
@@ -100,18 +94,67 @@ __device__ __forceinline__ bool pme_valid(const P4<CT>& r, double rx, double ry,
          fabs(y * ry) < 1e9 && fabs(z * rz) < 1e9;
 }
 
+// lanes per particle: order^2 (x, y) offsets rounded up to 16 or 64
+template <int ORDER>
+struct PmeLanes {
+  static constexpr int G = ORDER * ORDER <= 16 ? 16 : 64;
+};
+
+// Particles into bins of kPmeEdge^3 grid cells by the first cell of their
+// support, with max |q| and the rejected count of the call.  Slots are
+// claimed as the GSE binning claims them: one global atomic per workgroup
+// and touched bin, ranks within it from LDS (above kPmeAggBins bins, one per
+// particle: a workgroup's particles then touch most bins once).
+constexpr int kPmeEdge = 8, kPmeAggBins = 16384;
 template <typename CT>
-__global__ __launch_bounds__(256) void k_pme_qmax(const P4<CT>* __restrict__ xyzq, int n,
-                                                  double rx, double ry, double rz,
-                                                  BinStats* __restrict__ st) {
+__global__ __launch_bounds__(1024) void k_pme_bin(const P4<CT>* __restrict__ xyzq, int n,
+                                                  PmeGrid a, int cap, int agg,
+                                                  int* __restrict__ counts,
+                                                  BinStats* __restrict__ st,
+                                                  int* __restrict__ ovf,
+                                                  P4<CT>* __restrict__ sorted) {
+  extern __shared__ int pme_hist[];
+  __shared__ double wmax[16];
+  __shared__ int wbad[16];
+  const int i = blockIdx.x * 1024 + threadIdx.x;
+  if (agg)
+    for (int j = threadIdx.x; j < a.b.nbins; j += 1024) pme_hist[j] = 0;
+  __syncthreads();
+  int bin = -1, rank = 0, bad = 0;
   double qm = 0.0;
-  int bad = 0;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const P4<CT> r = xyzq[i];
-    if (pme_valid(r, rx, ry, rz))
-      qm = fmax(qm, fabs((double)r.w));
+  P4<CT> r{};
+  if (i < n) {
+    r = xyzq[i];
+    if (pme_valid(r, a.rx, a.ry, a.rz)) {
+      int ix, iy, iz;
+      double f;
+      pme_pos((double)r.x, a.rx, a.X, ix, f);
+      pme_pos((double)r.y, a.ry, a.Y, iy, f);
+      pme_pos((double)r.z, a.rz, a.Z, iz, f);
+      // a fraction rounded up to one counts as the first cell
+      ix = ix >= a.X ? ix - a.X : ix;
+      iy = iy >= a.Y ? iy - a.Y : iy;
+      iz = iz >= a.Z ? iz - a.Z : iz;
+      bin = ix / kPmeEdge + a.b.nbx * (iy / kPmeEdge + a.b.nby * (iz / kPmeEdge));
+      if (agg) rank = atomicAdd(&pme_hist[bin], 1);
+      qm = fabs((double)r.w);
+    } else {
+      bad = 1;
+    }
+  }
+  __syncthreads();
+  if (agg)
+    for (int j = threadIdx.x; j < a.b.nbins; j += 1024) {
+      const int c = pme_hist[j];
+      if (c > 0) pme_hist[j] = atomicAdd(&counts[j], c);
+    }
+  __syncthreads();
+  if (bin >= 0) {
+    const int slot = agg ? pme_hist[bin] + rank : atomicAdd(&counts[bin], 1);
+    if (slot < cap)
+      sorted[(size_t)bin * cap + slot] = r;
     else
-      bad++;
+      ovf[atomicAdd(&st->overflow, 1)] = i;
   }
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) {
@@ -119,55 +162,142 @@ __global__ __launch_bounds__(256) void k_pme_qmax(const P4<CT>* __restrict__ xyz
     bad += __shfl_xor(bad, m, kWave);
   }
   if ((threadIdx.x & 63) == 0) {
+    wmax[threadIdx.x >> 6] = qm;
+    wbad[threadIdx.x >> 6] = bad;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 16; w++) {
+      qm = fmax(qm, wmax[w]);
+      bad += wbad[w];
+    }
     if (qm > 0.0) atomicMax(&st->qmax_bits, (unsigned long long)__double_as_longlong(qm));
     if (bad) atomicAdd(&st->invalid, bad);
   }
 }
 
-// lanes per particle: order^2 (x, y) offsets rounded up to 16 or 64
-template <int ORDER>
-struct PmeLanes {
-  static constexpr int G = ORDER * ORDER <= 16 ? 16 : 64;
+// Spline of one axis per thread for a chunk of particles, in LDS: the lanes
+// of a particle share it.  (With every lane computing all three axes for
+// itself the order-6 spread and gather took 127 and 161 us for 200,001
+// charges on 125 x 126 x 128, 42 and 82 us with this.)
+constexpr int kPmeChunk = 64;
+template <int ORDER, bool DERIV>
+struct PmeSplines {
+  double th[kPmeChunk][3][ORDER];
+  double dth[DERIV ? kPmeChunk : 1][3][ORDER];
+  double q[kPmeChunk];  // charge; NaN marks a rejected particle
+  int cell[kPmeChunk][3];
 };
 
+// particle k of the chunk is load(k); 3 kPmeChunk threads; needs a barrier
+template <int ORDER, bool DERIV, typename CT, typename F>
+__device__ __forceinline__ void pme_splines(PmeSplines<ORDER, DERIV>& s, const PmeGrid& a, int cnt,
+                                            F load) {
+  const int k = threadIdx.x / 3, ax = threadIdx.x - 3 * k;
+  if (k >= cnt) return;
+  const P4<CT> r = load(k);
+  const bool ok = pme_valid(r, a.rx, a.ry, a.rz);
+  if (ax == 0) s.q[k] = ok ? (double)r.w : __builtin_nan("");
+  if (!ok) return;
+  const int M = ax == 0 ? a.X : ax == 1 ? a.Y : a.Z;
+  int c;
+  double f, th[ORDER], d[ORDER];
+  pme_pos((double)(ax == 0 ? r.x : ax == 1 ? r.y : r.z), ax == 0 ? a.rx : ax == 1 ? a.ry : a.rz, M,
+          c, f);
+  s.cell[k][ax] = c >= M ? c - M : c;  // a fraction rounded up to one: the first cell
+  pme_theta<ORDER>(f, th, d);
+#pragma unroll
+  for (int j = 0; j < ORDER; j++) {
+    s.th[k][ax][j] = th[j];
+    if (DERIV) s.dth[k][ax][j] = d[j];
+  }
+}
+
+// one lane's contributions of chunk particle k: offset (ax, ay) of its
+// support and every z offset; put(x, y, z, value) receives unwrapped cells
+template <int ORDER, typename F>
+__device__ __forceinline__ void pme_contrib(const PmeSplines<ORDER, false>& s, int k, double scale,
+                                            int ax, int ay, F put) {
+  // ((q tx) ty) tz as the reference orders it; the exact power-of-two
+  // scale changes no rounding
+  const double qxy = s.q[k] * scale * s.th[k][0][ax] * s.th[k][1][ay];
+  const int x = s.cell[k][0] + ax, y = s.cell[k][1] + ay, z = s.cell[k][2];
+#pragma unroll
+  for (int c = 0; c < ORDER; c++) put(x, y, z + c, fixed_round_prod(qxy, s.th[k][2][c]));
+}
+
+// B-spline spread of one bin per workgroup into an int64 brick in LDS
+// (kPmeEdge + ORDER - 1 cells a side), stored whole; k_brick_reduce adds the
+// bricks.  The kOverflowWG workgroups after the bins' add the particles that
+// found their bin full to the int64 grid with global atomics.  Spreading
+// every particle that way, 64 atomics of 8 bytes each to memory, took 49 us
+// of the 48,000-charge step at order 4, after 11 us for max |q|; binning,
+// spread and reduce take 5.7 + 10.3 + 8.4 (order 6, 200,001 charges on
+// 125 x 126 x 128: the whole step 870 -> 301 us).  The counts and the other
+// statistics buffer are cleared here for the next call.
 template <int ORDER, typename CT>
-__global__ __launch_bounds__(256) void k_pme_spread(const P4<CT>* __restrict__ xyzq, int n,
-                                                    int X, int Y, int Z, double rx, double ry,
-                                                    double rz, const BinStats* __restrict__ st,
-                                                    unsigned long long* __restrict__ g64) {
-  constexpr int G = PmeLanes<ORDER>::G;
-  constexpr int PER = 256 / G;
-  const int lane = threadIdx.x & (G - 1);
-  const int a = lane % ORDER, b = lane / ORDER;
+__global__ __launch_bounds__(256) void k_pme_spread(
+    const P4<CT>* __restrict__ xyzq, int n, PmeGrid a, int cap, int* __restrict__ counts,
+    const BinStats* __restrict__ st, BinStats* __restrict__ st_other,
+    const int* __restrict__ ovf, const P4<CT>* __restrict__ sorted, long long* __restrict__ bricks,
+    int* __restrict__ bshift, unsigned long long* __restrict__ g64) {
+  constexpr int G = PmeLanes<ORDER>::G, PER = 256 / G;
+  constexpr int L = kPmeEdge + ORDER - 1, VOL = L * L * L;
+  __shared__ unsigned long long brick[VOL];
+  __shared__ PmeSplines<ORDER, false> sp;
+  const int lane = threadIdx.x & (G - 1), ax = lane % ORDER, ay = lane / ORDER;
+  const bool live = lane < ORDER * ORDER;
   const BinStats s = *st;
   const double scale = ldexp(1.0, fixed_exponent(s.qmax_bits, n - s.invalid, 1, 1.0));
-  for (int p = blockIdx.x * PER + (int)(threadIdx.x / G); p < n; p += gridDim.x * PER) {
-    const P4<CT> r = xyzq[p];
-    if (!pme_valid(r, rx, ry, rz) || lane >= ORDER * ORDER) continue;
-    int ix, iy, iz;
-    double fx, fy, fz;
-    pme_pos((double)r.x, rx, X, ix, fx);
-    pme_pos((double)r.y, ry, Y, iy, fy);
-    pme_pos((double)r.z, rz, Z, iz, fz);
-    double tx[ORDER], ty[ORDER], tz[ORDER], d[ORDER];
-    pme_theta<ORDER>(fx, tx, d);
-    pme_theta<ORDER>(fy, ty, d);
-    pme_theta<ORDER>(fz, tz, d);
-    // ((q tx) ty) tz as the reference orders it; the exact power-of-two
-    // scale changes no rounding
-    const double qxy = (double)r.w * scale * tx[a] * ty[b];
-    int xi = ix + a, yi = iy + b;
-    if (xi >= X) xi -= X;
-    if (yi >= Y) yi -= Y;
-    const size_t row = (size_t)xi + (size_t)yi * X;
-#pragma unroll
-    for (int c = 0; c < ORDER; c++) {
-      int zi = iz + c;
-      if (zi >= Z) zi -= Z;
-      const long long v = fixed_round_prod(qxy, tz[c]);
-      atomicAdd(&g64[row + (size_t)zi * X * Y], (unsigned long long)v);
+  const int bin = blockIdx.x;
+  if (bin >= a.b.nbins) {
+    const int w = bin - a.b.nbins;
+    if (w == 0 && threadIdx.x == 0) {
+      st_other->qmax_bits = 0ull;
+      st_other->invalid = 0;
+      st_other->overflow = 0;
+      st_other->spill = 0;
     }
+    for (int k0 = w * kPmeChunk; k0 < s.overflow; k0 += kOverflowWG * kPmeChunk) {
+      const int m = min(kPmeChunk, s.overflow - k0);
+      pme_splines<ORDER, false, CT>(sp, a, m, [&](int k) { return xyzq[ovf[k0 + k]]; });
+      __syncthreads();
+      for (int k = threadIdx.x / G; k < m; k += PER)
+        if (live)
+          pme_contrib<ORDER>(sp, k, scale, ax, ay, [&](int x, int y, int z, long long v) {
+            x = x >= a.X ? x - a.X : x;
+            y = y >= a.Y ? y - a.Y : y;
+            z = z >= a.Z ? z - a.Z : z;
+            atomicAdd(&g64[x + (size_t)a.X * (y + (size_t)a.Y * z)], (unsigned long long)v);
+          });
+      __syncthreads();
+    }
+    return;
   }
+  const int cnt = min(counts[bin], cap);
+  for (int j = threadIdx.x; j < VOL; j += 256) brick[j] = 0ull;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    counts[bin] = 0;
+    bshift[bin] = cnt > 0 ? 0 : -1;
+  }
+  if (cnt == 0) return;
+  const int x0 = bin % a.b.nbx * kPmeEdge, y0 = bin / a.b.nbx % a.b.nby * kPmeEdge,
+            z0 = bin / (a.b.nbx * a.b.nby) * kPmeEdge;
+  for (int k0 = 0; k0 < cnt; k0 += kPmeChunk) {
+    const int m = min(kPmeChunk, cnt - k0);
+    pme_splines<ORDER, false, CT>(sp, a, m,
+                                  [&](int k) { return sorted[(size_t)bin * cap + k0 + k]; });
+    __syncthreads();
+    for (int k = threadIdx.x / G; k < m; k += PER)
+      if (live)
+        pme_contrib<ORDER>(sp, k, scale, ax, ay, [&](int x, int y, int z, long long v) {
+          atomicAdd(&brick[x - x0 + L * (y - y0 + L * (z - z0))], (unsigned long long)v);
+        });
+    __syncthreads();
+  }
+  for (int j = threadIdx.x; j < VOL; j += 256)
+    bricks[(size_t)bin * VOL + j] = (long long)brick[j];
 }
 
 struct PmeSum {
@@ -276,66 +406,56 @@ __global__ void __launch_bounds__(256)
 
 // CudaPMERecip.cu:1612-1890: dE/dr_a = q ccelec (M_a/L_a) sum dtheta_a theta
 // theta Qc; written times `sign` into out{x,y,z}[i].
+// Workgroups of `per` (at most kPmeChunk) consecutive particles.
 template <int ORDER, typename CT, typename AT>
 __global__ __launch_bounds__(256) void k_pme_gather(const P4<CT>* __restrict__ xyzq, int n,
-                                                    int X, int Y, int Z, double rx, double ry,
-                                                    double rz, double ccelec, double sign,
+                                                    PmeGrid g, int per, double ccelec, double sign,
                                                     const CT* __restrict__ Qc, AT* __restrict__ ox,
                                                     AT* __restrict__ oy, AT* __restrict__ oz) {
   constexpr int G = PmeLanes<ORDER>::G;
   constexpr int PER = 256 / G;
+  __shared__ PmeSplines<ORDER, true> sp;
   const int lane = threadIdx.x & (G - 1);
   const int a = lane % ORDER, b = lane / ORDER;
   const bool live = lane < ORDER * ORDER;
+  const int p0 = blockIdx.x * per, m = min(per, n - p0);
+  pme_splines<ORDER, true, CT>(sp, g, m, [&](int k) { return xyzq[p0 + k]; });
+  __syncthreads();
   // uniform trip count over the group so the butterfly sees every lane
-  const int pstart = blockIdx.x * PER + (int)(threadIdx.x / G);
-  const int nloop = (n + gridDim.x * PER - 1) / (gridDim.x * PER);
-  for (int it = 0; it < nloop; it++) {
-    const int p = pstart + it * gridDim.x * PER;
+  for (int k0 = 0; k0 < m; k0 += PER) {
+    const int k = k0 + (int)(threadIdx.x / G);
     CT f1 = 0, f2 = 0, f3 = 0;
-    bool ok = false;
-    P4<CT> r{};
-    if (p < n) {
-      r = xyzq[p];
-      ok = pme_valid(r, rx, ry, rz);
-    }
+    const double q = k < m ? sp.q[k] : 0.0;
+    const bool ok = k < m && q == q;
     if (ok && live) {
-      int ix, iy, iz;
-      double fx, fy, fz;
-      pme_pos((double)r.x, rx, X, ix, fx);
-      pme_pos((double)r.y, ry, Y, iy, fy);
-      pme_pos((double)r.z, rz, Z, iz, fz);
-      double tx[ORDER], ty[ORDER], tz[ORDER], dx[ORDER], dy[ORDER], dz[ORDER];
-      pme_theta<ORDER>(fx, tx, dx);
-      pme_theta<ORDER>(fy, ty, dy);
-      pme_theta<ORDER>(fz, tz, dz);
-      int xi = ix + a, yi = iy + b;
-      if (xi >= X) xi -= X;
-      if (yi >= Y) yi -= Y;
-      const CT* row = Qc + (size_t)xi + (size_t)yi * X;
-      const CT w1 = (CT)(dx[a] * ty[b]), w2 = (CT)(tx[a] * dy[b]), w3 = (CT)(tx[a] * ty[b]);
+      int xi = sp.cell[k][0] + a, yi = sp.cell[k][1] + b;
+      if (xi >= g.X) xi -= g.X;
+      if (yi >= g.Y) yi -= g.Y;
+      const CT* row = Qc + (size_t)xi + (size_t)yi * g.X;
+      const double tx = sp.th[k][0][a], ty = sp.th[k][1][b];
+      const CT w1 = (CT)(sp.dth[k][0][a] * ty), w2 = (CT)(tx * sp.dth[k][1][b]), w3 = (CT)(tx * ty);
 #pragma unroll
       for (int c = 0; c < ORDER; c++) {
-        int zi = iz + c;
-        if (zi >= Z) zi -= Z;
-        const CT g = row[(size_t)zi * X * Y];
-        const CT zc = (CT)tz[c], zd = (CT)dz[c];
-        f1 += w1 * zc * g;
-        f2 += w2 * zc * g;
-        f3 += w3 * zd * g;
+        int zi = sp.cell[k][2] + c;
+        if (zi >= g.Z) zi -= g.Z;
+        const CT v = row[(size_t)zi * g.X * g.Y];
+        const CT zc = (CT)sp.th[k][2][c], zd = (CT)sp.dth[k][2][c];
+        f1 += w1 * zc * v;
+        f2 += w2 * zc * v;
+        f3 += w3 * zd * v;
       }
     }
 #pragma unroll
-    for (int m = G / 2; m >= 1; m >>= 1) {
-      f1 += __shfl_xor(f1, m, kWave);
-      f2 += __shfl_xor(f2, m, kWave);
-      f3 += __shfl_xor(f3, m, kWave);
+    for (int i = G / 2; i >= 1; i >>= 1) {
+      f1 += __shfl_xor(f1, i, kWave);
+      f2 += __shfl_xor(f2, i, kWave);
+      f3 += __shfl_xor(f3, i, kWave);
     }
-    if (lane == 0 && p < n) {
-      const double q = ok ? (double)r.w * ccelec * sign : 0.0;
-      ox[p] = (AT)(q * rx * (double)f1 * X);
-      oy[p] = (AT)(q * ry * (double)f2 * Y);
-      oz[p] = (AT)(q * rz * (double)f3 * Z);
+    if (lane == 0 && k < m) {
+      const double s = ok ? q * ccelec * sign : 0.0;
+      ox[p0 + k] = (AT)(s * g.rx * (double)f1 * g.X);
+      oy[p0 + k] = (AT)(s * g.ry * (double)f2 * g.Y);
+      oz[p0 + k] = (AT)(s * g.rz * (double)f3 * g.Z);
     }
   }
 }
@@ -346,44 +466,68 @@ static unsigned blocks_for(long long count, unsigned threads, unsigned cap) {
   return (unsigned)(b < cap ? b : cap);
 }
 
-hipError_t launch_pme_qmax(bool dbl, const void* xyzq, int n, const double* recip3,
-                           BinStats* stats, hipStream_t s) {
-  k_clear_stats<<<1, 1, 0, s>>>(stats);
-  if (n <= 0) return hipGetLastError();
-  const unsigned grid = blocks_for(n, 256, 1024);
+PmeGrid pme_grid_make(int X, int Y, int Z, int order, const double* r) {
+  PmeGrid a;
+  a.X = X;
+  a.Y = Y;
+  a.Z = Z;
+  a.rx = r[0];
+  a.ry = r[1];
+  a.rz = r[2];
+  BinShape& b = a.b;
+  b.Bx = b.By = b.Bz = kPmeEdge;
+  b.nbx = (X + kPmeEdge - 1) / kPmeEdge;
+  b.nby = (Y + kPmeEdge - 1) / kPmeEdge;
+  b.nbz = (Z + kPmeEdge - 1) / kPmeEdge;
+  b.nbins = b.nbx * b.nby * b.nbz;
+  b.Lx = b.Ly = b.Lz = kPmeEdge + order - 1;
+  b.direct = 0;
+  return a;
+}
+
+hipError_t launch_pme_bin(bool dbl, const void* xyzq, int n, const PmeGrid& a, int cap,
+                          int* counts, BinStats* st, int* ovf, void* sorted, hipStream_t s) {
+  if (n <= 0) return hipSuccess;
+  const int agg = a.b.nbins <= kPmeAggBins ? 1 : 0;
+  const unsigned g = (unsigned)((n + 1023) / 1024);
+  const size_t lds = agg ? sizeof(int) * (size_t)a.b.nbins : 0;
   if (dbl)
-    k_pme_qmax<double><<<grid, 256, 0, s>>>((const P4<double>*)xyzq, n, recip3[0], recip3[1],
-                                            recip3[2], stats);
+    k_pme_bin<double><<<g, 1024, lds, s>>>((const P4<double>*)xyzq, n, a, cap, agg, counts, st,
+                                           ovf, (P4<double>*)sorted);
   else
-    k_pme_qmax<float><<<grid, 256, 0, s>>>((const P4<float>*)xyzq, n, recip3[0], recip3[1],
-                                           recip3[2], stats);
+    k_pme_bin<float><<<g, 1024, lds, s>>>((const P4<float>*)xyzq, n, a, cap, agg, counts, st, ovf,
+                                          (P4<float>*)sorted);
   return hipGetLastError();
 }
 
-template <int ORDER>
-static void pme_spread_o(bool dbl, const void* xyzq, int n, int X, int Y, int Z,
-                         const double* r, const BinStats* st, unsigned long long* g64,
+template <int ORDER, typename CT>
+static void pme_spread_t(const void* xyzq, int n, const PmeGrid& a, int cap, int* counts,
+                         const BinStats* st, BinStats* st_other, const int* ovf,
+                         const void* sorted, void* bricks, int* bshift, unsigned long long* g64,
                          hipStream_t s) {
-  constexpr int PER = 256 / PmeLanes<ORDER>::G;
-  const unsigned grid = blocks_for((n + PER - 1) / PER, 1, 8192);
-  if (dbl)
-    k_pme_spread<ORDER, double><<<grid, 256, 0, s>>>((const P4<double>*)xyzq, n, X, Y, Z, r[0],
-                                                     r[1], r[2], st, g64);
-  else
-    k_pme_spread<ORDER, float><<<grid, 256, 0, s>>>((const P4<float>*)xyzq, n, X, Y, Z, r[0],
-                                                    r[1], r[2], st, g64);
+  k_pme_spread<ORDER, CT><<<a.b.nbins + kOverflowWG, 256, 0, s>>>(
+      (const P4<CT>*)xyzq, n, a, cap, counts, st, st_other, ovf, (const P4<CT>*)sorted,
+      (long long*)bricks, bshift, g64);
 }
 
-hipError_t launch_pme_spread(bool dbl, int order, const void* xyzq, int n, int X, int Y, int Z,
-                             const double* recip3, const BinStats* stats,
+hipError_t launch_pme_spread(bool dbl, int order, const void* xyzq, int n, const PmeGrid& a,
+                             int cap, int* counts, const BinStats* st, BinStats* st_other,
+                             const int* ovf, const void* sorted, void* bricks, int* bshift,
                              unsigned long long* g64, hipStream_t s) {
-  if (n <= 0) return hipGetLastError();
+#define GSE_PME_SPREAD(O)                                                                      \
+  if (dbl)                                                                                     \
+    pme_spread_t<O, double>(xyzq, n, a, cap, counts, st, st_other, ovf, sorted, bricks, bshift, \
+                            g64, s);                                                           \
+  else                                                                                         \
+    pme_spread_t<O, float>(xyzq, n, a, cap, counts, st, st_other, ovf, sorted, bricks, bshift, \
+                           g64, s);
   switch (order) {
-    case 4: pme_spread_o<4>(dbl, xyzq, n, X, Y, Z, recip3, stats, g64, s); break;
-    case 6: pme_spread_o<6>(dbl, xyzq, n, X, Y, Z, recip3, stats, g64, s); break;
-    case 8: pme_spread_o<8>(dbl, xyzq, n, X, Y, Z, recip3, stats, g64, s); break;
+    case 4: GSE_PME_SPREAD(4) break;
+    case 6: GSE_PME_SPREAD(6) break;
+    case 8: GSE_PME_SPREAD(8) break;
     default: return hipErrorInvalidValue;
   }
+#undef GSE_PME_SPREAD
   return hipGetLastError();
 }
 
@@ -422,15 +566,18 @@ static void pme_gather_o(bool at_dbl, const void* xyzq, int n, int X, int Y, int
                          const double* r, double ccelec, double sign, const void* Qc, void* ox,
                          void* oy, void* oz, hipStream_t s) {
   constexpr int PER = 256 / PmeLanes<ORDER>::G;
-  const unsigned grid = blocks_for((n + PER - 1) / PER, 1, 8192);
+  // whole chunks once they still make four workgroups per CU
+  const int per = std::min(kPmeChunk, std::max(1, n / (1024 * PER)) * PER);
+  const unsigned grid = (unsigned)((n + per - 1) / per);
+  const PmeGrid g = pme_grid_make(X, Y, Z, ORDER, r);
   if (at_dbl)
-    k_pme_gather<ORDER, CT, double><<<grid, 256, 0, s>>>(
-        (const P4<CT>*)xyzq, n, X, Y, Z, r[0], r[1], r[2], ccelec, sign, (const CT*)Qc,
-        (double*)ox, (double*)oy, (double*)oz);
+    k_pme_gather<ORDER, CT, double><<<grid, 256, 0, s>>>((const P4<CT>*)xyzq, n, g, per, ccelec,
+                                                         sign, (const CT*)Qc, (double*)ox,
+                                                         (double*)oy, (double*)oz);
   else
-    k_pme_gather<ORDER, CT, float><<<grid, 256, 0, s>>>(
-        (const P4<CT>*)xyzq, n, X, Y, Z, r[0], r[1], r[2], ccelec, sign, (const CT*)Qc,
-        (float*)ox, (float*)oy, (float*)oz);
+    k_pme_gather<ORDER, CT, float><<<grid, 256, 0, s>>>((const P4<CT>*)xyzq, n, g, per, ccelec,
+                                                        sign, (const CT*)Qc, (float*)ox,
+                                                        (float*)oy, (float*)oz);
 }
 
 hipError_t launch_pme_gather(bool ct_dbl, bool at_dbl, int order, const void* xyzq, int n, int X,

@@ -202,6 +202,11 @@ hipError_t launch_brick_reduce(bool ct_double, bool acc32, const Geom& g, const 
                                const Binning& w, unsigned long long* grid64, void* out,
                                hipStream_t s);
 
+// the form for any bin shape and grid size
+hipError_t launch_brick_reduce_list(bool ct_double, bool acc32, const Geom& g, const BinShape& b,
+                                    const Binning& w, unsigned long long* grid64, void* out,
+                                    hipStream_t s);
+
 hipError_t launch_fill_u64(unsigned long long* p, size_t count, hipStream_t s);
 hipError_t launch_fill(bool dbl, void* p, size_t count, hipStream_t s);
 
@@ -449,13 +454,23 @@ hipError_t launch_charge_moments(bool dbl, const void* xyzq, int n,
                                  double* partials, hipStream_t s);
 
 // ---- SPME reciprocal comparator (ewald_pme.hip) -------------------------
-// recip3: 1/Lx, 1/Ly, 1/Lz.  stats: max |q| and the rejected count of the
-// call (cleared here), read by the spread and the int64 -> grid conversion.
 constexpr int kPmeSumBlocks = 512;
-hipError_t launch_pme_qmax(bool dbl, const void* xyzq, int n, const double* recip3,
-                           BinStats* stats, hipStream_t s);
-hipError_t launch_pme_spread(bool dbl, int order, const void* xyzq, int n, int X, int Y, int Z,
-                             const double* recip3, const BinStats* stats,
+// grid, reciprocal edges and bins of one spread (recip3: 1/Lx, 1/Ly, 1/Lz)
+struct PmeGrid {
+  int X, Y, Z;
+  double rx, ry, rz;
+  BinShape b;
+};
+PmeGrid pme_grid_make(int X, int Y, int Z, int order, const double* recip3);
+// bins: cap slots each in sorted [nbins * cap], counts [nbins] and st zero on
+// entry; the rest into ovf [n]
+hipError_t launch_pme_bin(bool dbl, const void* xyzq, int n, const PmeGrid& a, int cap,
+                          int* counts, BinStats* st, int* ovf, void* sorted, hipStream_t s);
+// bricks [nbins][L^3] int64 and bshift [nbins] for launch_brick_reduce_list,
+// overflow particles into g64; clears counts and st_other
+hipError_t launch_pme_spread(bool dbl, int order, const void* xyzq, int n, const PmeGrid& a,
+                             int cap, int* counts, const BinStats* st, BinStats* st_other,
+                             const int* ovf, const void* sorted, void* bricks, int* bshift,
                              unsigned long long* g64, hipStream_t s);
 // prefac: device [X + Y + Z] B-spline moduli; partials [kPmeSumBlocks][7]
 hipError_t launch_pme_scalar_sum(bool dbl, int X, int Y, int Z, const double* recip3,

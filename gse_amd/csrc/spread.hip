@@ -2584,6 +2584,12 @@ hipError_t launch_brick_reduce(bool dbl, bool acc32, const Geom& g, const BinSha
           w.pref_bound, grid64, (float*)out);
     return hipGetLastError();
   }
+  return launch_brick_reduce_list(dbl, acc32, g, b, w, grid64, out, s);
+}
+
+hipError_t launch_brick_reduce_list(bool dbl, bool acc32, const Geom& g, const BinShape& b,
+                                    const Binning& w, unsigned long long* grid64, void* out,
+                                    hipStream_t s) {
   const int nwg = (b.nbins + 7) / 8 * 8;
   // bricks that can cover one cell: those of the unwrapped axis, and one more
   // for each time a brick reaches round it (a last bin of under B cells)

@@ -113,6 +113,35 @@ def test_spme_fp32_water48k_force_rms():
         assert de <= 1e-5
 
 
+@pytest.mark.parametrize("order", [4, 6, 8])
+@pytest.mark.parametrize("dims", [(8, 9, 33), (16, 24, 20), (10, 8, 8)])
+def test_spme_bins_overflow_and_wrap(dims, order):
+    """The binned spread on grids of one to five bins per axis, last bins of
+    one to eight cells, bricks wrapping onto themselves, coordinates on box
+    faces, and a cluster that overfills its bin: the grid against the oracle,
+    and bit-identical for another order of the particles."""
+    rng = np.random.default_rng(order + dims[2])
+    box = tuple(1.1 * m for m in dims)
+    n = 700
+    x = np.empty((n, 4))
+    x[:, :3] = rng.random((n, 3)) * box
+    x[:400, :3] = 0.45 * np.array(box) + 0.3 * rng.random((400, 3))
+    x[400:403, :3] = [[0.0, 0.0, 0.0], list(box), [0.5 * box[0], 0.5 * box[1], 0.5 * box[2]]]
+    x[:, 3] = rng.standard_normal(n)
+    e, v, f = orc.pme_step(dims, order, x, box, 0.4)
+    pm = api.CudaPMERecip(F64, F64, *dims, order)
+    grids = []
+    for perm in (np.arange(n), rng.permutation(n), np.arange(n)):
+        pm.spread_charge(dev(x[perm]), n, box)
+        grids.append(pm.grid())
+    q = orc.pme_spread(dims, order, x, box)
+    assert rel(host(grids[0]), q) <= TOL
+    assert torch.equal(grids[0], grids[1]) and torch.equal(grids[0], grids[2])
+    o = pm.step(dev(x), box, 0.4)
+    assert abs(float(host(o["energy"])[0]) - e) <= TOL * abs(e)
+    assert rel(host(o["force"]).T, f) <= TOL
+
+
 def test_spme_bad_arguments():
     with pytest.raises(api._lib.GSEError):
         api.CudaPMERecip(F64, F64, 16, 16, 16, 5)

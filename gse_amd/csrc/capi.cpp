@@ -250,8 +250,8 @@ struct Engine {
       bin.bricks = bricks.p;
       bin.bshift = bshift.as<int>();
     }
-    spread_path = !g_tuning.spread_cols && g_tuning.spread_mma &&
-                          spread_mma_ok(ct_dbl, geom, shape, normalize, acc32(), brick_flush)
+    spread_path = !g_tuning.spread_cols && spread_mma_ok(ct_dbl, geom, shape, normalize, acc32(),
+                                                         brick_flush, bin.n)
                       ? 1
                       : 0;
     HIPCHK(launch_spread(ct_dbl, geom, shape, sigma, normalize, bin,
@@ -1020,7 +1020,7 @@ gse_status_t gse_set_tuning_param(const char* name, int value) {
   else if (n == "bin_order" && (value == 0 || value == 1)) t.bin_order = value;
   else if (n == "zpass4_cols" && (value == 0 || value == 16 || value == 32))
     t.zpass4_cols = value;
-  else if (n == "spread_mma" && (value == 0 || value == 1)) t.spread_mma = value;
+  else if (n == "spread_mma" && value >= 0 && value <= 2) t.spread_mma = value;
   else return fail(GSE_ERROR_INVALID_VALUE, "unknown tuning parameter or value out of range: %s=%d",
                    name, value);
   return GSE_SUCCESS;

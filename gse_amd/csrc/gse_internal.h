@@ -61,7 +61,7 @@ struct Tuning {
   int bin_coarse_block = 1024; // threads per super-bin binning workgroup (256, 512, 1024)
   int bin_order = 1;           // spread/gather workgroups take bins by descending count
   int gather_group = 32;       // lanes per charge in the FP32 13^3 gather walk (32, 16)
-  int spread_mma = 0;          // FP32 spread on the matrix cores (int8 limbs, exact sums)
+  int spread_mma = 2;          // FP32 spread on the matrix cores: 0 never, 1 always, 2 by occupancy
 };
 Tuning& tuning();
 // LDS bytes for the gather's staged particles (the gather_stage knob, or its
@@ -185,8 +185,9 @@ hipError_t launch_fixed_to_grid(bool ct_double, const unsigned long long* grid64
 constexpr size_t kBrickPad = 16;
 // Brick-store flush: usable for this shape (LDS path, bounded brick overlap)?
 bool brick_reduce_ok(const Geom& g, const BinShape& b);
+// n: charges of the call
 bool spread_mma_ok(bool dbl, const Geom& g, const BinShape& b, bool normalize, bool acc32,
-                   bool bricks);
+                   bool bricks, int n);
 // Which kernel converts a spread's fixed-point sums into the grid:
 enum ReducePath : int {
   kReduceAtomic = 0,   // bricks added with 64-bit atomics, then k_fixed_to_grid

@@ -969,166 +969,92 @@ __global__ void __launch_bounds__(BS, BS == 512 ? 6 : 1)
 // FP32 spread on the matrix cores.  Per bin the brick is a sum of outer
 // products,
 //   brick[(x, y), z] = sum_k A_k(x, y) B_k(z),
-//   A_k = round(q_k sA wx_k(x) wy_k(y)),  B_k = round(wz_k(z) kMmaSpan),
-// with sA = kMmaSpan / max|q|, so that |A| and B stay below kMmaSpan < 2^23,
-// each written as three signed 8-bit limbs (the limbs of v are the bytes of
-// (v + 0x808080) ^ 0x808080, v = l0 + 2^8 l1 + 2^16 l2).
-// v_mfma_i32_32x32x32_i8 sums the limb products over 32 particles per step:
-// rows are 32 (x, y) points of the brick plane, columns the z planes.  The
-// limb classes of weight 2^8 and above (li + lj >= 1) are summed exactly in
-// int32; l0 x l0 (below 2^14 per particle, against products up to 2^46) is
-// left out.  Every class sum is an exact integer sum, so the brick depends
+//   A_k = |q_k| sA wx_k(x) wy_k(y),  B_k = sign(q_k) wz_k(z) 2^22,
+// with sA the largest power of two that keeps A below kMmaSpan < 2^23 (so the
+// charges, a few values that all charges share, are not rounded by it), each
+// written as four signed 8-bit limbs, v = l0 + 2^8 l1 + 2^16 l2 + 2^-8 l3 (l3: the
+// rounding's remainder, by 254 instead of 256 so that it never reaches 128).
+// One multiply-add onto 2^23 + 0x8080 rounds the product to an integer and
+// leaves A + 0x8080 in the low bytes of the result: l0 and l1 are the first
+// two of them less 128 (one xor), l2 is the third.
+// v_mfma_i32_16x16x64_i8 sums the limb products over 64 particles per step:
+// rows are 16 (x, y) points of the brick plane, columns 16 z planes.  The
+// limb products of weight 2^8 and above are summed exactly in int32, the
+// smaller ones left out (below 2^15 per particle, against products up to
+// 2^46).  The fourth limbs matter although a brick value is rounded to 2^-24
+// of a charge: a factor's error is shared by a whole row or plane of cells,
+// and the potential sums those (with three limbs it was 1.9e-6 off at 48,000
+// charges, 1.6e-6 with every contribution rounded by itself, 6e-7 now).
+// Every class sum is an exact integer sum, so the brick depends
 // only on the set of particles whose home bin this is, not on their order:
 // the bin's overflow particles are taken from the overflow list and summed
 // into the same brick, and the int64 total is rounded once to the bin's
 // int32 scale 2^(e - shift), the scale and shift of the LDS-atomic path.
-// Operand layouts (measured): A lane l -> row l % 32, B lane l -> column
-// l % 32, and byte j of lane half l / 32 is the same k slot in A and B; the
-// 16 int32 results of lane l are rows 8 (r / 4) + 4 (l / 32) + r % 4, column
-// l % 32.
+//
+// Layout.  Four waves (eight on small grids) share the bin's 25 row tiles (25 x 16 = 20 x 20 points
+// exactly).  The factors go to LDS once as tables over (axis position,
+// particle), zero outside a particle's window, one lane per particle; a lane
+// then forms its row's A values of 16 consecutive particles from eight
+// 16-byte table reads and holds them as matrix operands without another trip
+// through LDS, and the results go from the accumulators to memory.  There is
+// no brick in LDS, so four workgroups share a CU and the 1000 bins of an 80^3
+// grid run at once.  The bound is VALU issue: seven instructions per A value,
+// eight per brick cell, and the chain from the counts to the tables.  Rows of the x and y tables are 132 floats apart: the
+// 16 x positions a 16-lane group reads fall on distinct 16-byte bank groups.
+// Measured at 80^3 / 48,000 charges and 216^3 / 1,000,002: 24.8 and 317 us,
+// against 32.4 and 437 us with LDS atomics; grid error against the FP64 oracle
+// 3.3e-7 of the largest value, against 1.34e-6.
+// Operand layouts: A lane l -> row l % 16, B lane l -> column l % 16, and
+// byte j of lane group l / 16 is the same particle in A and B; result r of
+// lane l is row 4 (l / 16) + r, column l % 16.
 // ---------------------------------------------------------------------------
 typedef int mma_v4i __attribute__((ext_vector_type(4)));
-typedef int mma_v16i __attribute__((ext_vector_type(16)));
 
 // Brick shape of the matrix-core spread: 2n+1 = 13 points per axis in bins
-// of 8 cells, so 20^3 bricks: 400 plane points in 13 row tiles of 32, 20 z
-// planes in one column tile of 32.
-constexpr int kMmaNZC = 13, kMmaLX = 20, kMmaLXY = 400, kMmaLZ = 20;
-constexpr int kMmaTiles = (kMmaLXY + 31) / 32;
-constexpr int kMmaThreads = 1024;     // 16 waves; waves below kMmaTiles own one row tile
-constexpr int kMmaK = 32;             // particles per MFMA step
-constexpr int kMmaMaxCall = 32768;    // int32 class sums stay exact below this
-constexpr int kMmaOvfWindow = kMmaThreads;
-constexpr float kMmaSpan = 8355000.0f;  // |A|, B below this: v + 0x808080 < 2^24
-constexpr int kMmaNW = 3 * kMmaNZC;
+// of 8 cells, so 20^3 bricks.
+constexpr int kMmaNZC = 13, kMmaL = 20, kMmaLXY = 400;
+constexpr int kMmaTiles = kMmaLXY / 16;  // row tiles
+constexpr int kMmaK = 128;            // particles in the tables (two MFMA steps)
+constexpr int kMmaPitch = kMmaK + 4;  // floats per x / y table row
+// the two highest classes are joined in int32: 2^8 sum l2 l2 + sum (l1 l2 +
+// l2 l1) <= (2^22 + 2^15) 500 < 2^31
+constexpr int kMmaMaxCall = 500;
+constexpr int kMmaOvfList = 512;      // overflow particles of one bin taken into its brick
+constexpr float kMmaSpan = 8355000.0f;   // A below this: A + 0x8080 < 2^23
+constexpr float kMmaSpanB = 4194304.0f;  // 2^22: |B| + 0x808080 < 2^24
+constexpr float kMmaMagic = 8388608.0f + 32896.0f;  // 2^23 + 0x8080
 
-// LDS layout: A table [kMmaK][kMmaLXY] packed limbs (the finished brick
-// reuses it), B limb bytes [3][32][kMmaK], factors [kMmaK][3 NZC], staged
-// particles, cube origins, scaled charges, overflow window and its count.
-constexpr int kMmaOA = 0;
-constexpr int kMmaOB = kMmaOA + kMmaK * kMmaLXY * 4;
-constexpr int kMmaOW = kMmaOB + 3 * 32 * kMmaK;
-constexpr int kMmaOP = (kMmaOW + kMmaK * kMmaNW * 4 + 15) & ~15;
-constexpr int kMmaOO = kMmaOP + kMmaK * 16;
-constexpr int kMmaOQ = kMmaOO + kMmaK * 4;
-constexpr int kMmaOL = kMmaOQ + kMmaK * 4;
-constexpr int kMmaON = kMmaOL + kMmaOvfWindow * 4;
-constexpr int kMmaLds = kMmaON + 16;
-static_assert(kMmaLXY * kMmaLZ <= kMmaK * kMmaLXY, "the brick fits the A table");
-static_assert(kMmaLds <= 64 * 1024, "LDS budget");
+struct MmaLds {
+  float x[kMmaL * kMmaPitch];      // q sA wx
+  float y[kMmaL * kMmaPitch];      // wy
+  alignas(16) unsigned char b[4][kMmaK / 64][32][64];  // limb bytes of wz: [limb][step][z][particle]
+  int ovf[kMmaOvfList];
+  int novf;
+};
 
-// bytes b of four packed-limb dwords -> one operand dword (byte t from d[t])
-__device__ __forceinline__ void mma_limbs4(unsigned d0, unsigned d1, unsigned d2, unsigned d3,
-                                           int& l0, int& l1, int& l2) {
-  const unsigned e01 = __builtin_amdgcn_perm(d1, d0, 0x05010400u);  // d0.b0 d1.b0 d0.b1 d1.b1
-  const unsigned e23 = __builtin_amdgcn_perm(d3, d2, 0x05010400u);
-  const unsigned f01 = __builtin_amdgcn_perm(d1, d0, 0x0c0c0602u);  // d0.b2 d1.b2 0 0
-  const unsigned f23 = __builtin_amdgcn_perm(d3, d2, 0x0c0c0602u);
-  l0 = (int)__builtin_amdgcn_perm(e23, e01, 0x05040100u);
-  l1 = (int)__builtin_amdgcn_perm(e23, e01, 0x07060302u);
+// the products of four particles -> one operand dword per limb (byte t from
+// particle t)
+__device__ __forceinline__ void mma_limbs4(const float4& u, const float4& v, int& l0, int& l1,
+                                           int& l2, int& l3) {
+  const float p[4] = {u.x, u.y, u.z, u.w}, w[4] = {v.x, v.y, v.z, v.w};
+  unsigned d[4], e[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const float f = __builtin_fmaf(p[k], w[k], kMmaMagic);
+    const float r = __builtin_fmaf(p[k], w[k], kMmaMagic - f);  // exact remainder
+    d[k] = __float_as_uint(f);
+    e[k] = __float_as_uint(__builtin_fmaf(r, 254.0f, 12582912.0f));  // 1.5 * 2^23
+  }
+  const unsigned e01 = __builtin_amdgcn_perm(d[1], d[0], 0x05010400u);  // d0.b0 d1.b0 d0.b1 d1.b1
+  const unsigned e23 = __builtin_amdgcn_perm(d[3], d[2], 0x05010400u);
+  const unsigned f01 = __builtin_amdgcn_perm(d[1], d[0], 0x0c0c0602u);  // d0.b2 d1.b2 0 0
+  const unsigned f23 = __builtin_amdgcn_perm(d[3], d[2], 0x0c0c0602u);
+  const unsigned g01 = __builtin_amdgcn_perm(e[1], e[0], 0x0c0c0400u);  // e0.b0 e1.b0 0 0
+  const unsigned g23 = __builtin_amdgcn_perm(e[3], e[2], 0x0c0c0400u);
+  l0 = (int)(__builtin_amdgcn_perm(e23, e01, 0x05040100u) ^ 0x80808080u);
+  l1 = (int)(__builtin_amdgcn_perm(e23, e01, 0x07060302u) ^ 0x80808080u);
   l2 = (int)__builtin_amdgcn_perm(f23, f01, 0x05040100u);
-}
-
-__device__ __forceinline__ unsigned mma_pack(int v) {
-  return ((unsigned)v + 0x808080u) ^ 0x808080u;
-}
-
-// One chunk of kc <= kMmaK staged particles (positions, cube origins and
-// scaled charges in LDS): factors, the A table and B operand, then the MFMA
-// steps of this wave's row tile.  Starts and ends with a barrier.
-__device__ __forceinline__ void mma_chunk(const SpreadArgs& a, int kc, unsigned char* lds,
-                                          mma_v16i (&acc)[4]) {
-  unsigned* sA = (unsigned*)(lds + kMmaOA);
-  signed char* sB = (signed char*)(lds + kMmaOB);
-  float* sW = (float*)(lds + kMmaOW);
-  const V4<float>* sP = (const V4<float>*)(lds + kMmaOP);
-  const int* sO = (const int*)(lds + kMmaOO);
-  const float* sQ = (const float*)(lds + kMmaOQ);
-  const int tid = threadIdx.x;
-  // the spacings as values first: a per-lane choice between fields of the
-  // argument struct would become an indexed copy of the struct in scratch
-  const double hx = a.g.hx, hy = a.g.hy, hz = a.g.hz;
-  const double ihx = a.g.ihx, ihy = a.g.ihy, ihz = a.g.ihz;
-  // factors, one thread per (particle, factor): t = (c h - x) + j h in FP64
-  // (CpuGaussCharge.cpp:314-329), the exponential in FP32
-  for (int e = tid; e < kc * kMmaNW; e += kMmaThreads) {
-    const int k = e / kMmaNW, f = e - k * kMmaNW;
-    const int axis = f / kMmaNZC, j = f - axis * kMmaNZC;
-    const V4<float> p = sP[k];
-    const double xv = axis == 0 ? (double)p.x : axis == 1 ? (double)p.y : (double)p.z;
-    const double h = axis == 0 ? hx : axis == 1 ? hy : hz;
-    const double ih = axis == 0 ? ihx : axis == 1 ? ihy : ihz;
-    const int c = (int)round(xv * ih) - (kMmaNZC - 1) / 2;
-    const double t = add_rn(sub_rn(mul_rn((double)c, h), xv), mul_rn((double)j, h));
-    const float tc = (float)t;
-    sW[e] = gexp(mul_rn(mul_rn(-tc, tc), (float)a.inv2s2));
-  }
-  // clear the A rows of the chunk's particles (16-byte stores)
-  {
-    uint4* a4 = (uint4*)sA;
-    for (int i = tid; i < kc * (kMmaLXY / 4); i += kMmaThreads) a4[i] = make_uint4(0u, 0u, 0u, 0u);
-  }
-  __syncthreads();
-  // A: one thread per (particle, y offset, half of the x offsets)
-  for (int e = tid; e < kc * kMmaNZC * 2; e += kMmaThreads) {
-    const int kr = e >> 1, hx = e & 1;
-    const int k = kr / kMmaNZC, dy = kr - k * kMmaNZC;
-    const int o = sO[k];
-    const float* w = sW + k * kMmaNW;
-    const float qy = sQ[k] * w[kMmaNZC + dy];
-    unsigned* row = sA + k * kMmaLXY + (o & 255) + kMmaLX * (((o >> 8) & 255) + dy);
-    const int dx0 = hx ? 7 : 0, dx1 = hx ? kMmaNZC : 7;
-#pragma unroll
-    for (int dx = 0; dx < 7; dx++)
-      if (dx0 + dx < dx1) row[dx0 + dx] = mma_pack((int)rintf(qy * w[dx0 + dx]));
-  }
-  // B: limb bytes [limb][z][slot]; zero outside the particle's z window and
-  // for slots past kc
-  for (int e = tid; e < 32 * kMmaK; e += kMmaThreads) {
-    const int z = e / kMmaK, k = e - z * kMmaK;
-    int v = 0;
-    if (k < kc && z < kMmaLZ) {
-      const int dz = z - (sO[k] >> 16);
-      if (dz >= 0 && dz < kMmaNZC) v = (int)rintf(sW[k * kMmaNW + 2 * kMmaNZC + dz] * kMmaSpan);
-    }
-    const unsigned pk = mma_pack(v);
-    sB[(0 * 32 + z) * kMmaK + k] = (signed char)(pk & 255u);
-    sB[(1 * 32 + z) * kMmaK + k] = (signed char)((pk >> 8) & 255u);
-    sB[(2 * 32 + z) * kMmaK + k] = (signed char)((pk >> 16) & 255u);
-  }
-  __syncthreads();
-  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  if (wid < kMmaTiles) {
-    const int lane = tid & 63, half = lane >> 5, col = lane & 31;
-    const mma_v4i b0 = *(const mma_v4i*)(sB + (0 * 32 + col) * kMmaK + 16 * half);
-    const mma_v4i b1 = *(const mma_v4i*)(sB + (1 * 32 + col) * kMmaK + 16 * half);
-    const mma_v4i b2 = *(const mma_v4i*)(sB + (2 * 32 + col) * kMmaK + 16 * half);
-    const int m = 32 * wid + col;
-    const unsigned* ak = sA + 16 * half * kMmaLXY + m;
-    unsigned d[16];
-#pragma unroll
-    for (int j = 0; j < 16; j++) d[j] = m < kMmaLXY ? ak[j * kMmaLXY] : 0u;
-    mma_v4i a0, a1, a2;
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      int l0, l1, l2;
-      mma_limbs4(d[4 * q], d[4 * q + 1], d[4 * q + 2], d[4 * q + 3], l0, l1, l2);
-      a0[q] = l0;
-      a1[q] = l1;
-      a2[q] = l2;
-    }
-    // limb classes of weight 2^8 (a0 b1 + a1 b0), 2^16 (a0 b2 + a1 b1 + a2 b0),
-    // 2^24 (a1 b2 + a2 b1) and 2^32 (a2 b2)
-    acc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, b1, acc[0], 0, 0, 0);
-    acc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, b0, acc[0], 0, 0, 0);
-    acc[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a0, b2, acc[1], 0, 0, 0);
-    acc[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, b1, acc[1], 0, 0, 0);
-    acc[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a2, b0, acc[1], 0, 0, 0);
-    acc[2] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, b2, acc[2], 0, 0, 0);
-    acc[2] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a2, b1, acc[2], 0, 0, 0);
-    acc[3] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a2, b2, acc[3], 0, 0, 0);
-  }
-  __syncthreads();
+  l3 = (int)__builtin_amdgcn_perm(g23, g01, 0x05040100u);
 }
 
 // Cube origin of a particle relative to its home bin (as k_bin stores it).
@@ -1139,166 +1065,286 @@ __device__ __forceinline__ int mma_origin(const Geom& g, const BinShape& b, cons
   return (ox % b.Bx) | ((oy % b.By) << 8) | ((oz % b.Bz) << 16);
 }
 
-// A bin with more than kMmaMaxCall particles: every one of them into the
-// int64 grid at the bin's scale, one wave per particle
-__device__ __forceinline__ void mma_giant_bin(
-    const SpreadArgs& a, const V4<float>* __restrict__ xyzq,
-    const V4<float>* __restrict__ sorted, const int* __restrict__ ovf, int novf, int bin,
-    int cnt, int eg, int shift, unsigned long long* __restrict__ grid64) {
-  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  constexpr int nwv = kMmaThreads / 64;
-  const double S = ldexp(1.0, eg - shift);
-  for (int i = wid; i < cnt; i += nwv)
-    spread_one_global<float>(a.g, a.inv2s2, a.pref, S, 0, a.pref1,
-                             sorted[(size_t)bin * a.cap_bin + i], grid64, shift);
-  for (int i = wid; i < novf; i += nwv) {
-    const V4<float> p = xyzq[ovf[i]];
-    if (home_bin<float>(a.g, a.b, p) == bin)
-      spread_one_global<float>(a.g, a.inv2s2, a.pref, S, 0, a.pref1, p, grid64, shift);
+// Tables of the particles c0 .. c0 + kc - 1 of a bin: its slots first, then
+// the collected overflow particles.  The tables are cleared, then each lane
+// writes one particle's factors at its window's positions; a wave takes ten
+// (five) of the 39 factors.  Needs a barrier before and after.
+template <int WAVES>
+__device__ __forceinline__ void mma_tables(const SpreadArgs& a, MmaLds& m, int c0, int kc, int cnt,
+                                           const V4<float>* __restrict__ slots,
+                                           const int* __restrict__ loc,
+                                           const V4<float>* __restrict__ xyzq, float qscale) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nks = (kc + 63) >> 6;
+  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int ks = 0; ks < nks; ks++) {
+    for (int e = threadIdx.x; e < kMmaL * 16; e += (64 * WAVES)) {
+      const int at = (e >> 4) * kMmaPitch + 64 * ks + 4 * (e & 15);
+      *(float4*)&m.x[at] = zero;
+      *(float4*)&m.y[at] = zero;
+    }
+    for (int e = threadIdx.x; e < 32 * 4; e += (64 * WAVES)) {
+      *(float4*)&m.b[0][ks][0][16 * e] = zero;
+      *(float4*)&m.b[1][ks][0][16 * e] = zero;
+      *(float4*)&m.b[2][ks][0][16 * e] = zero;
+      *(float4*)&m.b[3][ks][0][16 * e] = zero;
+    }
+  }
+  __syncthreads();
+  constexpr int per = (3 * kMmaNZC + WAVES - 1) / WAVES;
+  const int r0 = wave * per;
+  for (int ks = 0; ks < nks; ks++) {
+    const int k = 64 * ks + lane, i = c0 + k;
+    if (k >= kc) continue;
+    V4<float> p;
+    int o;
+    if (i < cnt) {
+      p = slots[i];
+      o = loc[i];
+    } else {
+      p = xyzq[m.ovf[i - cnt]];
+      o = mma_origin(a.g, a.b, p);
+    }
+#pragma unroll
+    for (int axis = 0; axis < 3; axis++) {
+      const int lo = max(0, r0 - kMmaNZC * axis), hi = min(kMmaNZC, r0 + per - kMmaNZC * axis);
+      if (lo >= hi) continue;
+      // factors: t = (c h - x) + j h in FP64 (CpuGaussCharge.cpp:314-329),
+      // the exponential in FP32
+      const double xv = axis == 0 ? (double)p.x : axis == 1 ? (double)p.y : (double)p.z;
+      const double h = axis == 0 ? a.g.hx : axis == 1 ? a.g.hy : a.g.hz;
+      const double ih = axis == 0 ? a.g.ihx : axis == 1 ? a.g.ihy : a.g.ihz;
+      const int c = (int)round(xv * ih) - (kMmaNZC - 1) / 2;
+      const double d0 = sub_rn(mul_rn((double)c, h), xv);
+      const int first = axis == 0 ? o & 255 : axis == 1 ? o >> 8 & 255 : o >> 16;
+      const float scale =
+          axis == 0 ? fabsf(p.w) * qscale : axis == 1 ? 1.0f : copysignf(kMmaSpanB, p.w);
+      for (int j = lo; j < hi; j++) {
+        const float tc = (float)add_rn(d0, mul_rn((double)j, h));
+        const float w = scale * gexp(mul_rn(mul_rn(-tc, tc), (float)a.inv2s2));
+        if (axis == 0) {
+          m.x[(first + j) * kMmaPitch + k] = w;
+        } else if (axis == 1) {
+          m.y[(first + j) * kMmaPitch + k] = w;
+        } else {
+          const float n = rintf(w);
+          const unsigned v = ((unsigned)(int)n + 0x808080u) ^ 0x808080u;
+          m.b[0][ks][first + j][lane] = (unsigned char)v;
+          m.b[1][ks][first + j][lane] = (unsigned char)(v >> 8);
+          m.b[2][ks][first + j][lane] = (unsigned char)(v >> 16);
+          m.b[3][ks][first + j][lane] = (unsigned char)(int)rintf((w - n) * 254.0f);
+        }
+      }
+    }
   }
 }
 
-// One workgroup per bin (no extra overflow workgroups: each bin sums its own
-// overflow particles).  A bin holding more than kMmaMaxCall particles takes
-// the per-contribution path instead: its particles go into the int64 grid at
-// its scale, as overflow particles of the LDS-atomic path do, and its brick
-// is marked empty.
-__global__ void __launch_bounds__(kMmaThreads)
+// A bin that holds more than its brick can take exactly: each of its slots'
+// particles into the int64 grid at the bin's scale, one wave per particle
+template <int WAVES>
+__device__ __forceinline__ void mma_giant_bin(const SpreadArgs& a,
+                                              const V4<float>* __restrict__ slots, int cnt,
+                                              int eg, int shift,
+                                              unsigned long long* __restrict__ grid64) {
+  const double S = ldexp(1.0, eg - shift);
+  for (int i = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); i < cnt; i += WAVES)
+    spread_one_global<float>(a.g, a.inv2s2, a.pref, S, 0, a.pref1, slots[i], grid64, shift);
+}
+__device__ __forceinline__ bool mma_giant(int call, int cap_bin) {
+  return call > kMmaMaxCall || call > cap_bin + kMmaOvfList;
+}
+
+// One bin: the brick of its `call` particles (cnt in slots, the rest on the
+// overflow list) and its shift, or, for a giant bin, its slots' particles in
+// the int64 grid and no brick.
+template <int WAVES>
+__device__ __forceinline__ void mma_bin(const SpreadArgs& a, MmaLds& m, int bin, int cnt, int call,
+                                        int eg, unsigned long long qbits, int novf,
+                                        const V4<float>* __restrict__ slots,
+                                        const int* __restrict__ loc,
+                                        const V4<float>* __restrict__ xyzq,
+                                        const int* __restrict__ ovf,
+                                        unsigned long long* __restrict__ grid64,
+                                        unsigned* __restrict__ brick, int* __restrict__ bshift) {
+  const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, grp = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ebin = fixed_exponent_bin(qbits, call, a.pref_bound);
+  const int shift = eg > ebin ? eg - ebin : 0;
+  const bool giant = mma_giant(call, a.cap_bin);
+  if (tid == 0) bshift[bin] = giant ? -1 : shift;
+  if (giant) {
+    mma_giant_bin<WAVES>(a, slots, cnt, eg, shift, grid64);
+    return;
+  }
+  // the total T = sum A B is q wx wy wz at the scale qscale kMmaSpanB and goes
+  // to the brick's q pref wx wy wz 2^(eg - shift), rounded once
+  union {
+    unsigned long long u;
+    double d;
+  } qv;
+  qv.u = qbits;
+  int eq = 0;
+  const double qm = frexp(qv.d, &eq);  // in [1/2, 1)
+  eq = qm * 8388608.0 < (double)kMmaSpan ? 23 - eq : 22 - eq;
+  const float qscale = qv.d > 0.0 ? (float)ldexp(1.0, eq) : 0.0f;
+  const double fct = qv.d > 0.0 ? ldexp(a.pref / (double)kMmaSpanB, eg - shift - eq) : 0.0;
+  const double f1 = fct * 256.0, f2 = fct * 65536.0, f3 = fct * 16777216.0;
+  if (call > cnt) {  // the bin's overflow particles, from the overflow list
+    if (tid == 0) m.novf = 0;
+    __syncthreads();
+    for (int i = tid; i < novf; i += (64 * WAVES)) {
+      const int pi = ovf[i];
+      if (home_bin<float>(a.g, a.b, xyzq[pi]) == bin) m.ovf[atomicAdd(&m.novf, 1)] = pi;
+    }
+    __syncthreads();
+  }
+  const bool once = call <= kMmaK;
+  if (once) {
+    mma_tables<WAVES>(a, m, 0, call, cnt, slots, loc, xyzq, qscale);
+    __syncthreads();
+  }
+  // exact class sums -> brick values at 2^(eg - shift): they convert to FP64
+  // exactly, the weighted sum is formed in a fixed order and rounded once (the
+  // same operations for any order of the particles)
+  auto put = [&](const mma_v4i(&acc)[4], unsigned at) {
+    unsigned r4[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      double v = (double)(acc[3][r] * 256 + acc[2][r]) * f3;
+      v = __builtin_fma((double)acc[1][r], f2, v);
+      v = __builtin_fma((double)acc[0][r], f1, v);
+      r4[r] = (unsigned)__double2loint(v + 6755399441055744.0);  // 1.5 * 2^52: rounds to nearest
+    }
+    *(uint4*)&brick[at] = make_uint4(r4[0], r4[1], r4[2], r4[3]);
+  };
+  // z planes 0..15 of a row tile fill one accumulator; planes 16..19 of four
+  // of the wave's tiles share another, tile q of the four in columns 4q..4q+3
+  // (its B operand is zero in the others: table column kMmaL)
+  mma_v4i top[4];
+#pragma unroll
+  for (int c = 0; c < 4; c++) top[c] = mma_v4i{0, 0, 0, 0};
+  constexpr int kRounds = (kMmaTiles + WAVES - 1) / WAVES;
+  for (int t = 0; t < kRounds; t++) {
+    const int tile = wave + WAVES * t, row = 16 * tile + l16;
+    const bool mine = tile < kMmaTiles;  // wave-uniform
+    const int y = row / kMmaL, x = row - y * kMmaL;
+    const int ctop = (l16 >> 2) == (t & 3) ? 16 + (l16 & 3) : kMmaL;
+    mma_v4i acc[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) acc[c] = mma_v4i{0, 0, 0, 0};
+    for (int c0 = 0; c0 < call; c0 += kMmaK) {
+      const int kc = min(kMmaK, call - c0);
+      if (!once) {  // more particles than the tables hold: rebuilt per row tile
+        __syncthreads();
+        mma_tables<WAVES>(a, m, c0, kc, cnt, slots, loc, xyzq, qscale);
+        __syncthreads();
+      }
+      for (int ks = 0; mine && 64 * ks < kc; ks++) {
+        const float4* px = (const float4*)&m.x[x * kMmaPitch + 64 * ks + 16 * grp];
+        const float4* py = (const float4*)&m.y[y * kMmaPitch + 64 * ks + 16 * grp];
+        mma_v4i a0, a1, a2, a3;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          int l0, l1, l2, l3;
+          mma_limbs4(px[q], py[q], l0, l1, l2, l3);
+          a0[q] = l0;
+          a1[q] = l1;
+          a2[q] = l2;
+          a3[q] = l3;
+        }
+        auto step = [&](mma_v4i(&d)[4], int col) {
+          const mma_v4i b0 = *(const mma_v4i*)&m.b[0][ks][col][16 * grp];
+          const mma_v4i b1 = *(const mma_v4i*)&m.b[1][ks][col][16 * grp];
+          const mma_v4i b2 = *(const mma_v4i*)&m.b[2][ks][col][16 * grp];
+          const mma_v4i b3 = *(const mma_v4i*)&m.b[3][ks][col][16 * grp];
+          // limb classes of weight 2^8 (a0 b1 + a1 b0 + a2 b3 + a3 b2), 2^16
+          // (a0 b2 + a1 b1 + a2 b0), 2^24 (a1 b2 + a2 b1) and 2^32 (a2 b2)
+          d[0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, b1, d[0], 0, 0, 0);
+          d[1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, b2, d[1], 0, 0, 0);
+          d[2] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, b2, d[2], 0, 0, 0);
+          d[3] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a2, b2, d[3], 0, 0, 0);
+          d[0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, b0, d[0], 0, 0, 0);
+          d[1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, b1, d[1], 0, 0, 0);
+          d[2] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a2, b1, d[2], 0, 0, 0);
+          d[0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a2, b3, d[0], 0, 0, 0);
+          d[1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a2, b0, d[1], 0, 0, 0);
+          d[0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a3, b2, d[0], 0, 0, 0);
+        };
+        step(acc, l16);
+        step(top, ctop);
+      }
+    }
+    if (mine) put(acc, 16 * tile + 4 * grp + kMmaLXY * l16);
+    if ((t & 3) == 3 || t == kRounds - 1) {
+      const int q = wave + WAVES * ((t & ~3) + (l16 >> 2));  // the tile of this column
+      if (q < kMmaTiles) put(top, 16 * q + 4 * grp + kMmaLXY * (16 + (l16 & 3)));
+#pragma unroll
+      for (int c = 0; c < 4; c++) top[c] = mma_v4i{0, 0, 0, 0};
+    }
+  }
+}
+
+// One workgroup per bin; kOverflowWG more add the overflow particles of giant
+// bins to the int64 grid.
+template <int WAVES>
+__global__ void __launch_bounds__(64 * WAVES, 4)
     k_spread_mma(SpreadArgs a, const V4<float>* __restrict__ xyzq,
                  const V4<float>* __restrict__ sorted, const int* __restrict__ counts,
                  int* __restrict__ counts_other, const BinStats* __restrict__ stats,
                  BinStats* __restrict__ stats_other, const int* __restrict__ ovf,
                  unsigned long long* __restrict__ grid64, unsigned* __restrict__ bricks,
                  int* __restrict__ bshift, const int* __restrict__ loc) {
-  extern __shared__ __align__(16) unsigned char mma_smem[];
+  __shared__ MmaLds m;
   const BinStats st = *stats;
   const int eg = fixed_exponent(st.qmax_bits, a.n - st.invalid, a.images, a.pref_bound);
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    stats_other->qmax_bits = 0ull;
-    stats_other->invalid = 0;
-    stats_other->overflow = 0;
-    stats_other->spill = 0;
+  if ((int)blockIdx.x >= a.nwg_bins) {
+    if (blockIdx.x == (unsigned)a.nwg_bins && threadIdx.x == 0) {
+      stats_other->qmax_bits = 0ull;
+      stats_other->invalid = 0;
+      stats_other->overflow = 0;
+      stats_other->spill = 0;
+    }
+    const int w = (int)blockIdx.x - a.nwg_bins;
+    const int gw = __builtin_amdgcn_readfirstlane(w * WAVES + (int)(threadIdx.x >> 6));
+    for (int k = gw; k < st.overflow; k += kOverflowWG * WAVES) {
+      const V4<float> p = xyzq[ovf[k]];
+      if (mma_giant(counts[home_bin<float>(a.g, a.b, p)], a.cap_bin))
+        spread_overflow<float, unsigned>(a, eg, st.qmax_bits, counts, p, grid64);
+    }
+    return;
   }
   const int pos = xcd_remap(blockIdx.x, a.nwg_bins);
   if (pos >= a.b.nbins) return;
   const int bin = bin_at(a.order, pos);
   const int call = counts[bin];
-  const int cnt = min(call, a.cap_bin);
   if (threadIdx.x == 0) {
     counts_other[bin] = 0;
-    if (call == 0 || call > kMmaMaxCall) bshift[bin] = -1;  // no brick this step
+    if (call == 0) bshift[bin] = -1;  // no brick this step
   }
   if (call == 0) return;
-  const Geom& g = a.g;
-  const BinShape& b = a.b;
-  const int ebin = fixed_exponent_bin(st.qmax_bits, call, a.pref_bound);
-  const int shift = eg > ebin ? eg - ebin : 0;
-  const int tid = threadIdx.x;
-  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-  if (call > kMmaMaxCall) {  // per-contribution path, one wave per particle
-    mma_giant_bin(a, xyzq, sorted, ovf, st.overflow, bin, cnt, eg, shift, grid64);
-    return;
-  }
-  // A = q qscale wx wy with qscale = kMmaSpan / qmax, so |A| <= kMmaSpan; the
-  // total T = sum A B is q wx wy wz at the scale qscale kMmaSpan and goes to
-  // the brick's q pref wx wy wz 2^(eg - shift), rounded once
-  union {
-    unsigned long long u;
-    double d;
-  } qv;
-  qv.u = st.qmax_bits;
-  const float qscale = qv.d > 0.0 ? (float)((double)kMmaSpan / qv.d) : 0.0f;
-  const double fct = qv.d > 0.0 ? ldexp(1.0, eg - shift) * a.pref /
-                                      ((double)qscale * (double)kMmaSpan)
-                                : 0.0;
-
-  unsigned char* lds = mma_smem;
-  V4<float>* sP = (V4<float>*)(lds + kMmaOP);
-  int* sO = (int*)(lds + kMmaOO);
-  float* sQ = (float*)(lds + kMmaOQ);
-  int* sL = (int*)(lds + kMmaOL);
-  int* sN = (int*)(lds + kMmaON);
-
-  mma_v16i acc[4];
-#pragma unroll
-  for (int c = 0; c < 4; c++)
-#pragma unroll
-    for (int r = 0; r < 16; r++) acc[c][r] = 0;
-
-  // the bin's slots
-  const V4<float>* bs = sorted + (size_t)bin * a.cap_bin;
-  const int* bl = loc + (size_t)bin * a.cap_bin;
-  for (int c0 = 0; c0 < cnt; c0 += kMmaK) {
-    const int kc = min(kMmaK, cnt - c0);
-    if (tid < kc) {
-      const V4<float> p = bs[c0 + tid];
-      sP[tid] = p;
-      sO[tid] = bl[c0 + tid];
-      sQ[tid] = p.w * qscale;
-    }
-    __syncthreads();
-    mma_chunk(a, kc, lds, acc);
-  }
-  // the bin's overflow particles, found on the overflow list a window at a time
-  if (call > cnt) {
-    for (int w0 = 0; w0 < st.overflow; w0 += kMmaOvfWindow) {
-      if (tid == 0) *sN = 0;
-      __syncthreads();
-      const int i = w0 + tid;
-      if (i < st.overflow) {
-        const int pi = ovf[i];
-        if (home_bin<float>(g, b, xyzq[pi]) == bin) sL[atomicAdd(sN, 1)] = pi;
-      }
-      __syncthreads();
-      const int nm = *sN;
-      __syncthreads();  // every thread has read the count before it is reset
-      for (int c0 = 0; c0 < nm; c0 += kMmaK) {
-        const int kc = min(kMmaK, nm - c0);
-        if (tid < kc) {
-          const V4<float> p = xyzq[sL[c0 + tid]];
-          sP[tid] = p;
-          sO[tid] = mma_origin(g, b, p);
-          sQ[tid] = p.w * qscale;
-        }
-        __syncthreads();
-        mma_chunk(a, kc, lds, acc);
-      }
-    }
-  }
-  // exact class sums -> the brick at 2^(eg - shift): each class sum converts
-  // to FP64 exactly, the weighted sum is formed in a fixed order and rounded
-  // once (the same operations for any order of the particles)
-  unsigned* sOut = (unsigned*)(lds + kMmaOA);
-  if (wid < kMmaTiles) {
-    const int lane = tid & 63, half = lane >> 5, col = lane & 31;
-    const double f1 = fct * 256.0, f2 = fct * 65536.0, f3 = fct * 16777216.0,
-                 f4 = fct * 4294967296.0;
-#pragma unroll
-    for (int r = 0; r < 16; r++) {
-      const int m = 32 * wid + 8 * (r >> 2) + 4 * half + (r & 3);
-      if (m < kMmaLXY && col < kMmaLZ) {
-        double v = (double)acc[3][r] * f4;
-        v = __builtin_fma((double)acc[2][r], f3, v);
-        v = __builtin_fma((double)acc[1][r], f2, v);
-        v = __builtin_fma((double)acc[0][r], f1, v);
-        sOut[m + kMmaLXY * col] = (unsigned)(int)rint(v);
-      }
-    }
-  }
-  __syncthreads();
-  constexpr int vol = kMmaLXY * kMmaLZ;
-  uint4* out = (uint4*)(bricks + (size_t)bin * vol);
-  for (int j = tid; j < vol / 4; j += kMmaThreads) out[j] = ((const uint4*)sOut)[j];
-  if (tid == 0) bshift[bin] = shift;
+  const size_t s0 = (size_t)bin * a.cap_bin;
+  mma_bin<WAVES>(a, m, bin, min(call, a.cap_bin), call, eg, st.qmax_bits, st.overflow, sorted + s0,
+          loc + s0, xyzq, ovf, grid64, bricks + (size_t)bin * (kMmaLXY * kMmaL), bshift);
 }
 
 // The matrix-core spread applies to FP32 grids with int32 bricks of
 // 20 x 20 x 20 (bins of 8 cells, 2n+1 = 13) and no normalisation.
 bool spread_mma_ok(bool dbl, const Geom& g, const BinShape& b, bool normalize, bool acc32,
-                   bool bricks) {
+                   bool bricks, int n) {
   if (dbl || !acc32 || !bricks || normalize || b.direct) return false;
   if (2 * g.nx + 1 != kMmaNZC || 2 * g.ny + 1 != kMmaNZC || 2 * g.nz + 1 != kMmaNZC) return false;
-  return b.Lx == kMmaLX && b.Ly * b.Lx == kMmaLXY && b.Lz == kMmaLZ;
+  if (b.Lx != kMmaL || b.Ly != kMmaL || b.Lz != kMmaL) return false;
+  // Automatic choice by the mean number of charges per bin.  A brick costs the
+  // matrix path the same from 1 to 64 charges and little more to 128, the LDS
+  // path in proportion to them; a bin past 128 rebuilds the tables for every
+  // row tile (30 us for the first, with a whole launch waiting for it).
+  // Measured, LDS / matrix us: 80^3 with 18 a bin 22.1 / 24.7, 24 25.4 / 25.0,
+  // 36 29.7 / 25.4, 48 34.8 / 26.0, 72 44.7 / 29.1, 96 54.0 / 61.0; 160^3 with
+  // 18 104 / 118, 24 115 / 118, 36 143 / 118, 72 242 / 160; 40^3 with 18 13.8 /
+  // 12.9, 72 23.8 / 15.5, 96 26.9 / 30.7.
+  const int knob = tuning().spread_mma;
+  return knob == 1 || (knob == 2 && n >= 24LL * b.nbins && n <= 72LL * b.nbins);
 }
 
 // Most bricks that may cover a cell along one axis (brick_reduce_ok).
@@ -2414,10 +2460,14 @@ static hipError_t spread_t(const Geom& g, const BinShape& b, double sigma, bool 
   }
   // stage as many particles as fit beside the brick in the workgroup's LDS
   const bool acc32 = sizeof(CT) == 4 && tu.spread_lds32;
-  if (tu.spread_mma && spread_mma_ok(sizeof(CT) == 8, g, b, normalize, acc32, w.bricks != nullptr)) {
-    a.cap = kMmaK;
+  if (spread_mma_ok(sizeof(CT) == 8, g, b, normalize, acc32, w.bricks != nullptr, w.n)) {
     a.nwg_bins = ((b.nbins + 7) / 8) * 8;
-    k_spread_mma<<<(unsigned)a.nwg_bins, kMmaThreads, kMmaLds, s>>>(
+    // eight waves a bin while every bin has a CU's matrix cores to itself or
+    // shares them with one other: the chain of row tiles sets the time there
+    // (32^3: 16.7 against 12.4 us, 54 x 63 x 50: 21.2 against 19.0); four give more bins at once beyond
+    const bool few = b.nbins <= 512;
+    (few ? k_spread_mma<8> : k_spread_mma<4>)<<<(unsigned)a.nwg_bins + kOverflowWG, few ? 512 : 256,
+                                               0, s>>>(
         a, (const V4<float>*)w.xyzq, (const V4<float>*)w.sorted, w.counts, w.counts_other,
         w.stats, w.stats_other, w.ovf, grid64, (unsigned*)w.bricks, w.bshift, w.loc);
     return hipGetLastError();

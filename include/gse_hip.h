@@ -119,7 +119,9 @@ GSE_API gse_status_t gse_set_tiling(int bin_edge, int lds_budget_bytes);
  *                 2D kernels measured faster at 64^2 to 128^2 planes)
  *   spread_mma    FP32 spreads with int32 bricks and a 13-point support run
  *                 on the matrix cores (int8 limb products summed exactly per
- *                 bin, the brick rounded once); 0 = LDS integer atomics (0/1, 0) */
+ *                 bin, the brick rounded once): 0 = never (LDS integer
+ *                 atomics), 1 = always, 2 = with 24 to 72 charges per bin on
+ *                 average, where it is the faster (0..2, 2) */
 GSE_API gse_status_t gse_set_tuning_param(const char* name, int value);
 GSE_API gse_status_t gse_get_tuning_param(const char* name, int* value);
 

@@ -722,7 +722,7 @@ def test_brick_reduce_any_shape(dims, h, dt, lds32):
     p = orc.Params(dims, box, 2.12)
     keys = api.get_tuning()
     try:
-        api.set_tuning(spread_lds32=lds32)
+        api.set_tuning(spread_lds32=lds32, spread_mma=0)  # one spread kernel for both flushes
         outs = []
         for flush, path in ((1, "generic"), (0, "atomic")):
             api.set_tuning(spread_flush=flush)
@@ -734,7 +734,8 @@ def test_brick_reduce_any_shape(dims, h, dt, lds32):
             outs.append(rho)
         assert torch.equal(outs[0], outs[1])
     finally:
-        api.set_tuning(spread_flush=keys["spread_flush"], spread_lds32=keys["spread_lds32"])
+        api.set_tuning(spread_flush=keys["spread_flush"], spread_lds32=keys["spread_lds32"],
+                       spread_mma=keys["spread_mma"])
 
 
 def test_numcoord_beyond_xyzq_is_rejected():

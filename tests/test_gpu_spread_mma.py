@@ -1,5 +1,5 @@
 """The FP32 spread on the matrix cores (int8 limb products summed exactly per
-bin, tuning knob spread_mma, off by default) against the FP64 oracle and
+bin, tuning knob spread_mma) against the FP64 oracle and
 against the LDS-atomic spread.
 
 The two FP32 kernels round differently (the matrix-core brick quantises the
@@ -111,8 +111,37 @@ def test_mma_spread_overflow_cluster():
     assert rel(host(r1), ref) <= 1e-6
 
 
+@pytest.mark.parametrize("extra", [1, 63, 64, 65, 127, 128, 129, 300, 600])
+def test_mma_spread_bin_counts(extra):
+    """Bins around one and two matrix steps, past the tables, and past the
+    exact class sums, on a grid with 2- and 7-cell last bins: within FP32 accuracy of
+    the oracle and bit-identical in any order.  A value is off by the
+    roundings of its bricks (half of 2^-30 of the bin's bound of extra
+    charges, at most 27 bricks) and by 2^-23 of each charge's factors."""
+    rng = np.random.default_rng(extra)
+    dims, box = (26, 31, 40), (26.0, 31.0, 40.0)
+    n = 400 + extra
+    xyzq = np.empty((n, 4))
+    xyzq[:, :3] = rng.random((n, 3)) * np.array(box)
+    xyzq[:extra, :3] = np.array([3.6, 4.6, 5.6]) + 2.0 * rng.random((extra, 3))
+    xyzq[:, 3] = rng.standard_normal(n)
+    p = orc.Params(dims, box, 2.12)
+    r1, lay = spread32(xyzq, p, True)
+    assert lay["spread"] == "mma"
+    perm = rng.permutation(n)
+    r2, _ = spread32(xyzq[perm], p, True)
+    assert torch.equal(r1, r2)
+    x32 = xyzq.astype(np.float32).astype(np.float64)
+    ref = orc.spread(p.dims, p.sigma1, p.rcut1, x32, p.box)
+    pref = (2 * np.pi * p.sigma1 ** 2) ** -1.5 * np.max(np.abs(x32[:, 3]))
+    bound = pref * (27 * 0.5 * 2.0 ** -30 * 2 * n + 2.0 ** -21 * np.sqrt(n))
+    err = np.max(np.abs(host(r1) - ref))
+    print(f"{extra}: err {err:.2e} bound {bound:.2e}", flush=True)
+    assert err <= bound
+
+
 def test_mma_spread_giant_bin_takes_the_per_contribution_path():
-    """A bin with more than 32768 particles is spread per contribution
+    """A bin with more than 500 particles is spread per contribution
     (int32 class sums would no longer be exact): with every particle in that
     bin, the grid is bit-identical to the LDS-atomic kernel's, which handles
     the same bin's overflow the same way."""

@@ -32,7 +32,7 @@ HBM_PEAK_GBS = 8000.0
 # profiles/k_gather_k_spread_water48k_M80_fp32_hbm_traffic.md.
 MEASURED_TRAFFIC = {
     ("water_48k_M80", "fp32", "gather"): 10650317,
-    ("water_48k_M80", "fp32", "spread"): 43789312,
+    ("water_48k_M80", "fp32", "spread"): 33052000,
 }
 # Wave-level VALU instructions per launch (rocprofv3 --pmc SQ_INSTS_VALU, same
 # file).  The gather and the spread issue far more vector instructions than
@@ -40,7 +40,7 @@ MEASURED_TRAFFIC = {
 # VALU instruction per CU per clock (4 SIMDs, 16 lanes each) = 614.4 G/s.
 MEASURED_VALU = {
     ("water_48k_M80", "fp32", "gather"): 15666063,
-    ("water_48k_M80", "fp32", "spread"): 8510291,
+    ("water_48k_M80", "fp32", "spread"): 8383947,
 }
 VALU_PEAK_GINST = 614.4
 

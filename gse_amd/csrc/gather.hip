@@ -121,7 +121,7 @@ __device__ void gather_one_global(const GatherArgs& a, const GatherOut& o, const
 
 // LDS layout of k_gather: staged 4-vectors (32-byte aligned) at 0, then the
 // factor pairs (w, d) of type CT, q (double), brick offsets and original
-// indices (int), then the potential brick (CT).
+// indices (int), then the potential brick (CT).  nw: pairs per charge.
 struct GatherLds {
   size_t oX, oW, oQ, oB, oP, oBrick, total;
 };
@@ -153,6 +153,11 @@ __host__ __device__ inline GatherLds gather_lds(int vol, int cap, int nw, int ct
 __host__ __device__ inline bool brick_v4(int ct_bytes, int X, int Bx) {
   return ct_bytes == 4 && X % 4 == 0 && Bx % 4 == 0;
 }
+// Factor pairs per charge of the FP32 two-charge walk with the virial sums: the
+// z axis has four
+// values per point, (wz, wz dz, rc^2 - dz^2, wz dz^2), at the front,
+// then (w, d) of the x and the y points.
+__host__ __device__ constexpr int pair_nw(int nzc) { return 4 * nzc; }
 __host__ __device__ inline int brick_pitch(int ct_bytes, int X, int Bx, int Lx) {
   return brick_v4(ct_bytes, X, Bx) ? (Lx + 3) & ~3 : Lx;
 }
@@ -180,7 +185,14 @@ __device__ __forceinline__ void gather_bin(const GatherArgs& a, int bin, int cnt
   const int Px = brick_pitch(sizeof(CT), g.X, b.Bx, Lx), PxLy = Px * Ly;
   const int NX = 2 * g.nx + 1, NY = 2 * g.ny + 1;
   const int NZ = NZC > 0 ? NZC : 2 * g.nz + 1;
-  const int NW = NX + NY + NZ;
+  // the FP32 paired walk with the virial keeps four values per z point: the
+  // products are formed once per charge instead of by every lane (54 x 63 x 50,
+  // 16,239 charges: 30.5 -> 26.8 us).  Without the virial the two-value table
+  // and one wave per charge are faster (80^3, 48,000 charges: 33.8 against
+  // 35.0 us), the larger tables costing more LDS traffic than they save.
+  constexpr bool ZTAB =
+      NZC > 0 && sizeof(CT) == 4 && sizeof(AT) == 4 && PL > 0 && (FL & GF_VIRIAL) != 0;
+  const int NW = ZTAB ? pair_nw(NZC) : NX + NY + NZ;
   const int cap = a.cap;
   const GatherLds lay = gather_lds(PxLy * Lz, cap, NW, sizeof(CT));
   char* lds = (char*)smem_raw;
@@ -206,7 +218,7 @@ __device__ __forceinline__ void gather_bin(const GatherArgs& a, int bin, int cnt
      // thread has that many in flight instead of one.  Wrapped grid rows come
      // from two small tables (Ly, Lz <= 64: the brick may be wider than the
      // grid, so one conditional wrap would not do).
-    __shared__ int s_gy[64], s_gz[64];
+    __shared__ int s_gx[64], s_gy[64], s_gz[64];
     if (threadIdx.x < (unsigned)Ly) {
       int v = byi * b.By + (int)threadIdx.x;
       while (v >= g.Y) v -= g.Y;
@@ -215,12 +227,18 @@ __device__ __forceinline__ void gather_bin(const GatherArgs& a, int bin, int cnt
       int v = bzi * b.Bz + (int)threadIdx.x - 64;
       while (v >= g.Z) v -= g.Z;
       s_gz[threadIdx.x - 64] = v;
+    } else if (threadIdx.x >= 128 && threadIdx.x < 192) {  // 16-byte pieces of a row
+      s_gx[threadIdx.x - 128] = (((bxi * b.Bx) >> 2) + (int)threadIdx.x - 128) % max(g.X >> 2, 1);
     }
     __syncthreads();
-    constexpr int kStageBatch = 8;
+    // 20 x 20 x 20 bricks are 2000 16-byte pieces, 24 x 22 x 22 are 2904: one
+    // batch of 4 or 6 per thread, with the wrapped piece of a row from a table
+    // (80^3, 48,000 charges: 34.4 -> 33.8 us against a batch of 8 with its
+    // second half idle and an integer remainder per piece)
+    constexpr int kStageBatch = BS == 512 && PL == 400 ? 4 : BS == 512 && PL == 528 ? 6 : 8;
     if (sizeof(CT) == 4 && brick_v4(4, g.X, b.Bx)) {
       // 16-byte pieces: row r = ly + Ly*lz, piece j covers columns 4j..4j+3
-      const int nq = Px >> 2, xq = g.X >> 2, gq0 = (bxi * b.Bx) >> 2;
+      const int nq = Px >> 2, xq = g.X >> 2;
       const int total = Ly * Lz * nq;
       const float inv_nq = 1.0f / (float)nq, inv_ly = 1.0f / (float)Ly;
       for (int e0 = threadIdx.x; e0 < total; e0 += kStageBatch * BS) {
@@ -235,9 +253,8 @@ __device__ __forceinline__ void gather_bin(const GatherArgs& a, int bin, int cnt
           int lz = (int)(((float)row + 0.5f) * inv_ly);
           const int ly = row - lz * Ly;
           lz = lz < Lz ? lz : Lz - 1;
-          const int qx = (gq0 + j) % xq;
           dst[u] = ok ? Px * row + 4 * j : -1;
-          v[u] = ok ? ((const float4*)phi)[qx + (size_t)xq * (s_gy[ly] + (size_t)g.Y * s_gz[lz])]
+          v[u] = ok ? ((const float4*)phi)[s_gx[j] + (size_t)xq * (s_gy[ly] + (size_t)g.Y * s_gz[lz])]
                     : make_float4(0.f, 0.f, 0.f, 0.f);
         }
 #pragma unroll
@@ -333,7 +350,7 @@ __device__ __forceinline__ void gather_bin(const GatherArgs& a, int bin, int cnt
   // FP64 pairs too (without the virial sums, whose extra z tables would not
   // fit beside two charges' registers), with the reference's exact test
   constexpr bool PAIR = FMA_FORM && PL > 0 && (sizeof(CT) == 4 || !VIR);
-  constexpr bool EXACT_SPH = VIR || sizeof(CT) == 8;
+  constexpr bool EXACT_SPH = sizeof(CT) == 8;
   // GS lanes per charge (32: two charges per wave; 16: four)
   static_assert(GS == 32 || GS == 16, "charge groups of 32 or 16 lanes");
   constexpr int GPW = 64 / GS;
@@ -390,6 +407,29 @@ __device__ __forceinline__ void gather_bin(const GatherArgs& a, int bin, int cnt
         sW[2 * e] = gexp(mul_rn(mul_rn(-d, d), inv2s2));
         sW[2 * e + 1] = d;
       }
+    } else if constexpr (ZTAB) {
+      // FP32, cubic support: one axis of 64 consecutive (charge, point)
+      // entries per wave, so the axis is uniform and every lane has an entry
+      const int nch = (na * NZA + 63) >> 6;
+      for (int t = wid; t < 3 * nch; t += nwv) {
+        const int ax = (t >= nch) + (t >= 2 * nch);
+        const int e = (t - ax * nch) * 64 + lane;
+        const double hs = ax == 0 ? hx_u : ax == 1 ? hy_u : hz_u;
+        const double ihs = ax == 0 ? ihx_u : ax == 1 ? ihy_u : ihz_u;
+        if (e < na * NZA) {
+          const int ai = e / NZA, j = e - ai * NZA;
+          const double ps = (double)((const CT*)sX)[4 * ai + ax];
+          const int c = (int)round(ps * ihs);
+          const CT d = (CT)sub_rn(ps, mul_rn((double)(c - gnz + j), hs));
+          const CT d2 = mul_rn(d, d);
+          const CT wt = gexp(mul_rn(-d2, inv2s2));
+          CT* w = sW + (size_t)ai * NW * 2;
+          if (ax == 2)
+            ((V4<CT>*)w)[j] = V4<CT>{wt, wt * d, rc2 - d2, wt * d2};
+          else
+            *(float2*)&w[4 * NZA + 2 * (ax * NZA + j)] = make_float2(wt, d);
+        }
+      }
     } else {
       for (int ai = wid; ai < na; ai += nwv) {
         const V4<CT> p = sX[ai];
@@ -414,16 +454,21 @@ __device__ __forceinline__ void gather_bin(const GatherArgs& a, int bin, int cnt
         const int aic = live ? ai : GPW * g2;
         const CT* w = sW + (size_t)aic * NW * 2;
         const int base = sB[aic];
-        // dz2: rc^2 - dz^2 (no virial: one compare per point), else dz^2
-        // (the virial weight, and the exact sphere test); w2r = wz dz^2
+        // dz2: rc^2 - dz^2 (one compare per point), FP64: dz^2 (the exact
+        // sphere test); w2r = wz dz^2
         CT wzr[NZA], dz2[NZA], vzr[NZA], w2r[VIR ? NZA : 1];
 #pragma unroll
         for (int t = 0; t < NZA; t++) {
+          if constexpr (ZTAB) {
+            const V4<CT> z = ((const V4<CT>*)w)[t];
+            wzr[t] = z.x, vzr[t] = z.y, dz2[t] = z.z;
+            if constexpr (VIR) w2r[t] = z.w;
+            continue;
+          }
           wzr[t] = w[2 * (2 * NZA + t)];
           const CT dz = w[2 * (2 * NZA + t) + 1];
           dz2[t] = EXACT_SPH ? mul_rn(dz, dz) : rc2 - mul_rn(dz, dz);
           vzr[t] = wzr[t] * dz;
-          if constexpr (VIR) w2r[t] = wzr[t] * dz2[t];
         }
         AT f[13];
 #pragma unroll
@@ -431,10 +476,11 @@ __device__ __forceinline__ void gather_bin(const GatherArgs& a, int bin, int cnt
 #pragma unroll
         for (int k = 0; k < KP; k++) {
           if (l32 + GS * k >= NXYP) continue;
-          const CT wx = w[2 * p_tx[k]];
-          const CT dx = w[2 * p_tx[k] + 1];
-          const CT wy = w[2 * (NZA + p_ty[k])];
-          const CT dy = w[2 * (NZA + p_ty[k]) + 1];
+          const CT* wxy_t = w + (ZTAB ? 4 * NZA : 0);
+          const CT wx = wxy_t[2 * p_tx[k]];
+          const CT dx = wxy_t[2 * p_tx[k] + 1];
+          const CT wy = wxy_t[2 * (NZA + p_ty[k])];
+          const CT dy = wxy_t[2 * (NZA + p_ty[k]) + 1];
           const CT dxy2 = add_rn(mul_rn(dx, dx), mul_rn(dy, dy));
           const int a0 = base + p_tx[k] + Px * p_ty[k];
           AT B0 = 0, B1 = 0, B2 = 0, A0 = 0, A1 = 0;
@@ -451,7 +497,7 @@ __device__ __forceinline__ void gather_bin(const GatherArgs& a, int bin, int cnt
               A1 = fmac((AT)vzr[t], (AT)ph, A1);
             } else if (SPH && cl == 0) {
               // (dx^2 + dy^2) + dz^2 < rc^2 as CpuGaussCharge.cpp:157 rounds
-              // it (FP64, virial), else dx^2 + dy^2 < rc^2 - dz^2
+              // it (FP64), else dx^2 + dy^2 < rc^2 - dz^2
               const bool in = EXACT_SPH ? add_rn(dxy2, dz2[t]) < rc2 : dxy2 < dz2[t];
               const AT ms = in ? (AT)ph : (AT)0;
               A0 = fmac((AT)wzr[t], ms, A0);
@@ -906,10 +952,22 @@ static hipError_t gather_nz(GatherArgs a, const Binning& w, const void* phi, con
                                                      w.stats_other, ph, o);
     return hipGetLastError();
   }
-  const int NW = 2 * (a.g.nx + a.g.ny + a.g.nz) + 3;
-  const int vol = brick_pitch(sizeof(CT), a.g.X, a.b.Bx, a.b.Lx) * a.b.Ly * a.b.Lz;
   const Tuning& tu = tuning();
-  const size_t lds_total = (size_t)vol * sizeof(CT) + (size_t)gather_stage_bytes(sizeof(CT) == 8);
+  const int bs = tu.gather_block ? tu.gather_block : (sizeof(CT) == 4 ? 512 : 256);
+  const int pxly = brick_pitch(sizeof(CT), a.g.X, a.b.Bx, a.b.Lx) * a.b.Ly;
+  // 8^3 bins with n = 6 on every axis: 20 x 20 planes of the brick (FP32;
+  // not the full output set, whose sums do not fit the register budget)
+  const bool pair13 = sizeof(CT) == 4 && FL != (GF_SPHERE | GF_CUBE | GF_POT | GF_VIRIAL) &&
+                      bs == 512 && pxly == 400 && a.g.nz == 6 && a.g.nx == a.g.nz &&
+                      a.g.ny == a.g.nz;
+  const bool ztab = pair13 && sizeof(AT) == 4 && (FL & GF_VIRIAL) != 0;
+  const int NW = ztab ? pair_nw(13) : 2 * (a.g.nx + a.g.ny + a.g.nz) + 3;
+  const int vol = pxly * a.b.Lz;
+  // four-value tables are 416 bytes a charge: what two workgroups per CU leave
+  // beside the 32 KB brick, so that a bin's charges are one chunk
+  const size_t stage = ztab && !tu.gather_stage ? (size_t)(46 * 1024)
+                                                : (size_t)gather_stage_bytes(sizeof(CT) == 8);
+  const size_t lds_total = (size_t)vol * sizeof(CT) + stage;
   int cap = 256;
   while (cap > 1 && gather_lds(vol, cap, NW, sizeof(CT)).total > lds_total) cap--;
   a.cap = cap;
@@ -920,7 +978,6 @@ static hipError_t gather_nz(GatherArgs a, const Binning& w, const void* phi, con
   a.order_next = w.order_next;
   a.order_wg0 = a.nwg_bins + kOverflowWG + (o.fin_partials ? 1 : 0);
   const unsigned nwg = (unsigned)(a.order_wg0 + (a.order_next ? kOrderWG : 0));
-  const int bs = tu.gather_block ? tu.gather_block : (sizeof(CT) == 4 ? 512 : 256);
 #define GSE_G_ARGS a, xq, srt, w.perm, w.counts, w.counts_other, w.stats, w.stats_other, w.ovf, ph, o, \
                    w.loc
 #define GSE_G_BS(NZV)                                                      \
@@ -928,14 +985,11 @@ static hipError_t gather_nz(GatherArgs a, const Binning& w, const void* phi, con
     k_gather<CT, AT, NZV, FL, 512><<<nwg, 512, lds, s>>>(GSE_G_ARGS);     \
   else                                                                     \
     k_gather<CT, AT, NZV, FL, 256><<<nwg, 256, lds, s>>>(GSE_G_ARGS);
-  const int pxly = brick_pitch(sizeof(CT), a.g.X, a.b.Bx, a.b.Lx) * a.b.Ly;
   switch (2 * a.g.nz + 1) {
     case 11: GSE_G_BS(11) break;
     case 13:
-      // 8^3 bins with n = 6 on every axis: 20 x 20 planes of the brick (FP32;
-      // not the full output set, whose sums do not fit the register budget)
       if constexpr (sizeof(CT) == 4 && FL != (GF_SPHERE | GF_CUBE | GF_POT | GF_VIRIAL)) {
-        if (bs == 512 && pxly == 400 && a.g.nx == a.g.nz && a.g.ny == a.g.nz) {
+        if (pair13) {
           if (tu.gather_group == 16)
             k_gather<CT, AT, 13, FL, 512, 400, 16><<<nwg, 512, lds, s>>>(GSE_G_ARGS);
           else
@@ -969,6 +1023,9 @@ static hipError_t gather_fl(int flags, const GatherArgs& a, const Binning& w, co
   if ((flags & ~(S | P)) == 0) return gather_nz<CT, AT, S | P>(a, w, phi, o, s);
   if ((flags & ~(C | P)) == 0) return gather_nz<CT, AT, C | P>(a, w, phi, o, s);
   if ((flags & ~(C | P | V)) == 0) return gather_nz<CT, AT, C | P | V>(a, w, phi, o, s);
+  // without the cube force the virial's sums fit the paired walk's registers
+  // (54 x 63 x 50, 16,239 charges: 47.6 us with all thirteen sums, 26.8 here)
+  if ((flags & ~(S | P | V)) == 0) return gather_nz<CT, AT, S | P | V>(a, w, phi, o, s);
   return gather_nz<CT, AT, S | C | P | V>(a, w, phi, o, s);
 }
 

@@ -127,6 +127,36 @@ def test_gather_cube_potential_virial_fp64(case):
     assert rel(host(o["virial"]).reshape(3, 3), vir) <= TOL
 
 
+@pytest.mark.parametrize("dims", [(32, 40, 32), (30, 33, 35)], ids=["aligned", "ragged"])
+@pytest.mark.parametrize("n,dense", [(1, 0), (3, 0), (700, 0), (900, 123)])
+@pytest.mark.parametrize("flags", [9, 13])
+def test_gather_sphere_virial_fp32(dims, n, dense, flags):
+    """Sphere force with the virial (and the potential) in FP32: one and three
+    charges (a wave's second half without a charge), and a bin of more charges
+    than one staged chunk.  Bound: a term w(d) phi d is off by about 8 * 2^-24 of
+    itself (its offset, exponential and products), and with a random phi the sum
+    of the absolute terms is about sqrt(120) * 0.8 = 9 times the result's size,
+    120 = (sqrt(4 pi) sigma / h)^3 points: 4.3e-6."""
+    X, Y, Z = dims
+    box = tuple(0.97 * m for m in dims)
+    rng = np.random.default_rng(n + dense)
+    x = np.empty((n, 4))
+    x[:, :3] = rng.random((n, 3)) * box
+    x[:dense, :3] = 0.97 * (8.5 + 7 * rng.random((dense, 3)))  # inside one bin of 8 cells
+    x[:, 3] = rng.standard_normal(n)
+    x = x.astype(np.float32).astype(np.float64)
+    p = orc.Params(dims, box, 2.12)
+    phi = rng.normal(size=(Z, Y, X)).astype(np.float32).astype(np.float64)
+    g = api.CpuGaussCharge(F32, F32, *dims)
+    o = g.gather(p.sigma1, p.rcut1, to_dev(x, F32), p.box, to_dev(phi, F32), flags)
+    pot, _, vir = orc.gather_cube(p.dims, p.sigma1, p.rcut1, x, p.box, phi)
+    ref = orc.interpolate(p.dims, p.sigma1, p.rcut1, x, p.box, phi)
+    assert rel(host(o["force"]).T, ref) <= 4.3e-6
+    assert rel(host(o["virial"]).reshape(3, 3), vir) <= 4.3e-6
+    if flags & 4:
+        assert rel(host(o["pot"]), pot) <= 4.3e-6
+
+
 # ---------------------------------------------------------- k-space
 @pytest.mark.parametrize("kind,sigma", [(0, 0.9487), (0, 0.0), (1, 0.9487)])
 @pytest.mark.parametrize("dims,box", [((20, 20, 20), (20.0,) * 3), ((18, 16, 24), (18.0, 16.2, 21.6)),

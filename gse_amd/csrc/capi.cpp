@@ -801,8 +801,10 @@ struct gse_pme_recip_s {
   int n_last = 0;
   KSolverFFTOnly* fft = nullptr;
   DevBuf grid64, grid, spec, prefac, partials, stats, tmp2, counts, ovf, sorted, bricks, bshift;
-  int cur = 0;         // the statistics buffer of the next spread
-  bool clean = false;  // counts and that buffer are zero
+  // counts and stats[0] are zero between calls: create clears them and every
+  // call's kernels leave them so.  Once a call failed halfway, each later one
+  // clears them itself (a captured call may not be run before the next one)
+  bool dirty = false;
   hipStream_t stream = nullptr;
 };
 
@@ -1873,7 +1875,10 @@ gse_status_t gse_pme_recip_create(gse_pme_recip_t* out, gse_dtype_t at, gse_dtyp
   h->fft = new KSolverFFTOnly();
   const size_t np = (size_t)nfftx * nffty * nfftz;
   const size_t nk = (size_t)(nfftx / 2 + 1) * nffty * nfftz;
+  const double unit[3] = {1.0, 1.0, 1.0};
+  const int nb = pme_grid_make(nfftx, nffty, nfftz, order, unit).b.nbins;
   gse_status_t st = h->fft->fft.init(h->ct_dbl, nfftx, nffty, nfftz);
+  if (st == GSE_SUCCESS) st = h->counts.ensure(sizeof(int) * (size_t)nb);
   if (st == GSE_SUCCESS) st = h->grid64.ensure(8 * np);
   if (st == GSE_SUCCESS) st = h->grid.ensure(tsize(h->ct_dbl) * np);
   if (st == GSE_SUCCESS) st = h->spec.ensure(2 * tsize(h->ct_dbl) * nk);
@@ -1889,6 +1894,8 @@ gse_status_t gse_pme_recip_create(gse_pme_recip_t* out, gse_dtype_t at, gse_dtyp
     hipError_t e = hipMemcpy(h->prefac.p, pf.data(), sizeof(double) * pf.size(),
                              hipMemcpyHostToDevice);
     if (e == hipSuccess) e = launch_fill_u64(h->grid64.as<unsigned long long>(), np, nullptr);
+    if (e == hipSuccess)
+      e = launch_bin_clear(h->counts.as<int>(), nb, h->stats.as<BinStats>(), nullptr);
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     if (e != hipSuccess) st = fail(GSE_ERROR_HIP, "SPME set-up failed: %s", hipGetErrorString(e));
   }
@@ -1932,31 +1939,29 @@ gse_status_t gse_pme_recip_spread_charge(gse_pme_recip_t h, const void* xyzq, in
   // twice the mean occupancy plus a margin; the rest spreads by itself
   const int nb = a.b.nbins, cap = (int)((2LL * ncoord / nb + 32 + 15) / 16 * 16);
   const size_t vol = (size_t)a.b.Lx * a.b.Ly * a.b.Lz;
-  GSECHK(h->counts.ensure(sizeof(int) * (size_t)nb));
   GSECHK(h->bshift.ensure(sizeof(int) * (size_t)nb));
   GSECHK(h->bricks.ensure(8 * vol * nb + kBrickPad));
   GSECHK(h->sorted.ensure(4 * tsize(h->ct_dbl) * (size_t)nb * cap));
   GSECHK(h->ovf.ensure(sizeof(int) * (size_t)std::max(ncoord, 1)));
-  BinStats* st = h->stats.as<BinStats>() + h->cur;
-  if (!h->clean) HIPCHK(launch_bin_clear(h->counts.as<int>(), nb, st, s));
-  h->clean = false;
+  BinStats *st = h->stats.as<BinStats>(), *kept = st + 1;
+  const bool dirty = h->dirty;
+  h->dirty = true;
+  if (dirty) HIPCHK(launch_bin_clear(h->counts.as<int>(), nb, st, s));
   HIPCHK(launch_pme_bin(h->ct_dbl, xyzq, ncoord, a, cap, h->counts.as<int>(), st,
                         h->ovf.as<int>(), h->sorted.p, s));
   HIPCHK(launch_pme_spread(h->ct_dbl, h->order, xyzq, ncoord, a, cap, h->counts.as<int>(), st,
-                           h->stats.as<BinStats>() + (h->cur ^ 1), h->ovf.as<int>(), h->sorted.p,
-                           h->bricks.p, h->bshift.as<int>(), h->grid64.as<unsigned long long>(),
-                           s));
+                           kept, h->ovf.as<int>(), h->sorted.p, h->bricks.p,
+                           h->bshift.as<int>(), h->grid64.as<unsigned long long>(), s));
   Binning w;
   w.n = ncoord;
-  w.stats = st;
+  w.stats = kept;
   w.pref_bound = 1.0;
   w.bricks = h->bricks.p;
   w.bshift = h->bshift.as<int>();
   const Geom g = make_geom(h->X, h->Y, h->Z, 1.0, 1.0, 1.0, 1.0);
   HIPCHK(launch_brick_reduce_list(h->ct_dbl, false, g, a.b, w, h->grid64.as<unsigned long long>(),
-                                  h->grid.p, s));
-  h->cur ^= 1;
-  h->clean = true;
+                                  h->grid.p, s, st));
+  h->dirty = dirty;
   return GSE_SUCCESS;
 }
 

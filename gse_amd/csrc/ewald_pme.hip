@@ -233,12 +233,14 @@ __device__ __forceinline__ void pme_contrib(const PmeSplines<ORDER, false>& s, i
 // every particle that way, 64 atomics of 8 bytes each to memory, took 49 us
 // of the 48,000-charge step at order 4, after 11 us for max |q|; binning,
 // spread and reduce take 5.7 + 10.3 + 8.4 (order 6, 200,001 charges on
-// 125 x 126 x 128: the whole step 870 -> 301 us).  The counts and the other
-// statistics buffer are cleared here for the next call.
+// 125 x 126 x 128: the whole step 870 -> 301 us).  The counts are cleared here
+// by their only reader; st_kept receives the statistics for k_brick_reduce,
+// which clears st.  A call so leaves counts and st zero, with no host state
+// that a replay of its captured launches would not change.
 template <int ORDER, typename CT>
 __global__ __launch_bounds__(256) void k_pme_spread(
     const P4<CT>* __restrict__ xyzq, int n, PmeGrid a, int cap, int* __restrict__ counts,
-    const BinStats* __restrict__ st, BinStats* __restrict__ st_other,
+    const BinStats* __restrict__ st, BinStats* __restrict__ st_kept,
     const int* __restrict__ ovf, const P4<CT>* __restrict__ sorted, long long* __restrict__ bricks,
     int* __restrict__ bshift, unsigned long long* __restrict__ g64) {
   constexpr int G = PmeLanes<ORDER>::G, PER = 256 / G;
@@ -252,12 +254,7 @@ __global__ __launch_bounds__(256) void k_pme_spread(
   const int bin = blockIdx.x;
   if (bin >= a.b.nbins) {
     const int w = bin - a.b.nbins;
-    if (w == 0 && threadIdx.x == 0) {
-      st_other->qmax_bits = 0ull;
-      st_other->invalid = 0;
-      st_other->overflow = 0;
-      st_other->spill = 0;
-    }
+    if (w == 0 && threadIdx.x == 0) *st_kept = s;
     for (int k0 = w * kPmeChunk; k0 < s.overflow; k0 += kOverflowWG * kPmeChunk) {
       const int m = min(kPmeChunk, s.overflow - k0);
       pme_splines<ORDER, false, CT>(sp, a, m, [&](int k) { return xyzq[ovf[k0 + k]]; });
@@ -502,24 +499,24 @@ hipError_t launch_pme_bin(bool dbl, const void* xyzq, int n, const PmeGrid& a, i
 
 template <int ORDER, typename CT>
 static void pme_spread_t(const void* xyzq, int n, const PmeGrid& a, int cap, int* counts,
-                         const BinStats* st, BinStats* st_other, const int* ovf,
+                         const BinStats* st, BinStats* st_kept, const int* ovf,
                          const void* sorted, void* bricks, int* bshift, unsigned long long* g64,
                          hipStream_t s) {
   k_pme_spread<ORDER, CT><<<a.b.nbins + kOverflowWG, 256, 0, s>>>(
-      (const P4<CT>*)xyzq, n, a, cap, counts, st, st_other, ovf, (const P4<CT>*)sorted,
+      (const P4<CT>*)xyzq, n, a, cap, counts, st, st_kept, ovf, (const P4<CT>*)sorted,
       (long long*)bricks, bshift, g64);
 }
 
 hipError_t launch_pme_spread(bool dbl, int order, const void* xyzq, int n, const PmeGrid& a,
-                             int cap, int* counts, const BinStats* st, BinStats* st_other,
+                             int cap, int* counts, const BinStats* st, BinStats* st_kept,
                              const int* ovf, const void* sorted, void* bricks, int* bshift,
                              unsigned long long* g64, hipStream_t s) {
 #define GSE_PME_SPREAD(O)                                                                      \
   if (dbl)                                                                                     \
-    pme_spread_t<O, double>(xyzq, n, a, cap, counts, st, st_other, ovf, sorted, bricks, bshift, \
+    pme_spread_t<O, double>(xyzq, n, a, cap, counts, st, st_kept, ovf, sorted, bricks, bshift, \
                             g64, s);                                                           \
   else                                                                                         \
-    pme_spread_t<O, float>(xyzq, n, a, cap, counts, st, st_other, ovf, sorted, bricks, bshift, \
+    pme_spread_t<O, float>(xyzq, n, a, cap, counts, st, st_kept, ovf, sorted, bricks, bshift,  \
                            g64, s);
   switch (order) {
     case 4: GSE_PME_SPREAD(4) break;

@@ -203,10 +203,10 @@ hipError_t launch_brick_reduce(bool ct_double, bool acc32, const Geom& g, const 
                                const Binning& w, unsigned long long* grid64, void* out,
                                hipStream_t s);
 
-// the form for any bin shape and grid size
+// the form for any bin shape and grid size; `clear` (not w.stats) is zeroed
 hipError_t launch_brick_reduce_list(bool ct_double, bool acc32, const Geom& g, const BinShape& b,
                                     const Binning& w, unsigned long long* grid64, void* out,
-                                    hipStream_t s);
+                                    hipStream_t s, BinStats* clear = nullptr);
 
 hipError_t launch_fill_u64(unsigned long long* p, size_t count, hipStream_t s);
 hipError_t launch_fill(bool dbl, void* p, size_t count, hipStream_t s);
@@ -468,9 +468,9 @@ PmeGrid pme_grid_make(int X, int Y, int Z, int order, const double* recip3);
 hipError_t launch_pme_bin(bool dbl, const void* xyzq, int n, const PmeGrid& a, int cap,
                           int* counts, BinStats* st, int* ovf, void* sorted, hipStream_t s);
 // bricks [nbins][L^3] int64 and bshift [nbins] for launch_brick_reduce_list,
-// overflow particles into g64; clears counts and st_other
+// overflow particles into g64; clears counts, copies st to st_kept
 hipError_t launch_pme_spread(bool dbl, int order, const void* xyzq, int n, const PmeGrid& a,
-                             int cap, int* counts, const BinStats* st, BinStats* st_other,
+                             int cap, int* counts, const BinStats* st, BinStats* st_kept,
                              const int* ovf, const void* sorted, void* bricks, int* bshift,
                              unsigned long long* g64, hipStream_t s);
 // prefac: device [X + Y + Z] B-spline moduli; partials [kPmeSumBlocks][7]

@@ -1379,13 +1379,14 @@ __global__ void __launch_bounds__(BT)
     k_brick_reduce(Geom g, BinShape b, int nwg, const ACC* __restrict__ bricks,
                    const int* __restrict__ bshift, const BinStats* __restrict__ stats, int n,
                    int images, double pref_bound, unsigned long long* __restrict__ grid64,
-                   T* __restrict__ out) {
+                   T* __restrict__ out, BinStats* __restrict__ clear) {
   constexpr int NE = 16 / (int)sizeof(ACC), UN = 12;
   extern __shared__ __align__(16) unsigned char reduce_smem[];
   BrickRef* list = (BrickRef*)reduce_smem;
   __shared__ int axis_bin[3 * KR], axis_cell[3 * KR];
   __shared__ int nlist;
   const int tile = xcd_remap(blockIdx.x, nwg);
+  if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = BinStats{};
   if (tile >= b.nbins) return;
   const BinStats st = *stats;
   const int cx = tile % b.nbx, cy = (tile / b.nbx) % b.nby, cz = tile / (b.nbx * b.nby);
@@ -2639,7 +2640,7 @@ hipError_t launch_brick_reduce(bool dbl, bool acc32, const Geom& g, const BinSha
 
 hipError_t launch_brick_reduce_list(bool dbl, bool acc32, const Geom& g, const BinShape& b,
                                     const Binning& w, unsigned long long* grid64, void* out,
-                                    hipStream_t s) {
+                                    hipStream_t s, BinStats* clear) {
   const int nwg = (b.nbins + 7) / 8 * 8;
   // bricks that can cover one cell: those of the unwrapped axis, and one more
   // for each time a brick reaches round it (a last bin of under B cells)
@@ -2649,15 +2650,15 @@ hipError_t launch_brick_reduce_list(bool dbl, bool acc32, const Geom& g, const B
   if (dbl)
     k_brick_reduce<double, unsigned long long, 256><<<nwg, 256, lds, s>>>(
         g, b, nwg, (const unsigned long long*)w.bricks, w.bshift, w.stats, w.n, w.images,
-        w.pref_bound, grid64, (double*)out);
+        w.pref_bound, grid64, (double*)out, clear);
   else if (acc32)
     k_brick_reduce<float, unsigned, 128><<<nwg, 128, lds, s>>>(
         g, b, nwg, (const unsigned*)w.bricks, w.bshift, w.stats, w.n, w.images, w.pref_bound, grid64,
-        (float*)out);
+        (float*)out, clear);
   else
     k_brick_reduce<float, unsigned long long, 256><<<nwg, 256, lds, s>>>(
         g, b, nwg, (const unsigned long long*)w.bricks, w.bshift, w.stats, w.n, w.images,
-        w.pref_bound, grid64, (float*)out);
+        w.pref_bound, grid64, (float*)out, clear);
   return hipGetLastError();
 }
 

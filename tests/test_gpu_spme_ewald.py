@@ -142,6 +142,53 @@ def test_spme_bins_overflow_and_wrap(dims, order):
     assert rel(host(o["force"]).T, f) <= TOL
 
 
+def spme_uneven(n, box, seed):
+    """Particles of which most share two cells, with some that are rejected."""
+    rng = np.random.default_rng(seed)
+    x = np.empty((n, 4))
+    x[:, :3] = rng.random((n, 3)) * box
+    x[: n // 2, :3] = (0.2 + 0.1 * seed) * np.array(box) + 0.3 * rng.random((n // 2, 3))
+    x[:, 3] = rng.standard_normal(n)
+    x[n // 3 : n // 3 + 5 * (seed % 3), seed % 4] = np.nan
+    return x
+
+
+def test_spme_captured_step_replays_like_the_eager_one():
+    """A captured step of an unevenly filled box, replayed with the positions
+    (and the number of rejected particles) changed in between and with eager
+    calls of another size on the same handle, against a fresh handle's eager
+    step: the same bits.  No count may be carried from one replay to the
+    next, for overfull bins and rejected particles would add up."""
+    dims, box, n = (24, 18, 33), (24.0, 18.0, 33.0), 900
+    x = dev(spme_uneven(n, box, 0), F32)
+    other = dev(spme_uneven(300, box, 5), F32)
+    pm = api.CudaPMERecip(F32, F32, *dims, 4)
+    o = pm.step(x, box, 0.4)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        pm.step(x, box, 0.4, out=o)
+    for seed in range(6):
+        x.copy_(dev(spme_uneven(n, box, seed), F32))
+        graph.replay()
+        ref = api.CudaPMERecip(F32, F32, *dims, 4)
+        r = ref.step(x, box, 0.4)
+        torch.cuda.synchronize()
+        for k in ("energy", "virial", "force"):
+            assert torch.equal(o[k], r[k]), (seed, k)
+        if seed % 2:
+            pm.spread_charge(other, len(other), box)
+            ref.spread_charge(other, len(other), box)
+            assert torch.equal(pm.grid(), ref.grid())
+    # captured and never replayed: the next eager step is unaffected
+    unused = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(unused):
+        pm.spread_charge(x, n, box)
+    pm.spread_charge(x, n, box)
+    ref.spread_charge(x, n, box)
+    assert torch.equal(pm.grid(), ref.grid())
+
+
 def test_spme_bad_arguments():
     with pytest.raises(api._lib.GSEError):
         api.CudaPMERecip(F64, F64, 16, 16, 16, 5)

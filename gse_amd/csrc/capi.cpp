@@ -800,7 +800,9 @@ struct gse_pme_recip_s {
   double recip3[3] = {0, 0, 0};  // of the last spread (gather and scalar_sum reuse it)
   int n_last = 0;
   KSolverFFTOnly* fft = nullptr;
-  DevBuf grid64, grid, spec, prefac, partials, stats, tmp2, counts, ovf, sorted, bricks, bshift;
+  DevBuf grid64, grid, spec, prefac, partials, stats, tmp2, counts, bricks, bshift;
+  DevBuf slots;                  // the bins' particles, then the overflow list
+  std::vector<DevBuf> outgrown;  // smaller `slots` of before: a captured call may still use them
   // counts and stats[0] are zero between calls: create clears them and every
   // call's kernels leave them so.  Once a call failed halfway, each later one
   // clears them itself (a captured call may not be run before the next one)
@@ -1848,7 +1850,35 @@ gse_status_t pme_recip3(const double* recip, double* r3) {
   return GSE_SUCCESS;
 }
 
-// the int64 -> grid conversion reads max |q| and the count from a Binning
+// slots per bin for n particles: twice the mean occupancy plus a margin; the
+// rest spreads by itself
+int pme_cap(int n, int nb) { return (int)((2LL * n / nb + 32 + 15) / 16 * 16); }
+size_t pme_sorted_bytes(bool dbl, int n, int nb) {
+  return 4 * tsize(dbl) * (size_t)nb * pme_cap(n, nb);
+}
+size_t pme_slot_bytes(bool dbl, int n, int nb) {
+  return pme_sorted_bytes(dbl, n, nb) + sizeof(int) * (size_t)n;
+}
+
+// Larger slots, at least twice the size.  Only more particles than any call
+// before come here, so that may be a call under stream capture: the
+// allocation is no part of the graph, and what earlier graphs use is kept.
+gse_status_t pme_grow_slots(gse_pme_recip_s* h, size_t need) {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  HIPCHK(hipThreadExchangeStreamCaptureMode(&mode));
+  DevBuf b;
+  gse_status_t st = b.ensure(std::max(need, 2 * h->slots.bytes));
+  if (st != GSE_SUCCESS) {
+    (void)hipGetLastError();
+    st = b.ensure(need);
+  }
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  GSECHK(st);
+  if (h->slots.p) h->outgrown.push_back(h->slots);
+  h->slots = b;
+  return GSE_SUCCESS;
+}
+
 constexpr double kPmeCcelec = 332.0716;  // CudaPMERecip.h:25
 
 }  // namespace
@@ -1876,9 +1906,15 @@ gse_status_t gse_pme_recip_create(gse_pme_recip_t* out, gse_dtype_t at, gse_dtyp
   const size_t np = (size_t)nfftx * nffty * nfftz;
   const size_t nk = (size_t)(nfftx / 2 + 1) * nffty * nfftz;
   const double unit[3] = {1.0, 1.0, 1.0};
-  const int nb = pme_grid_make(nfftx, nffty, nfftz, order, unit).b.nbins;
+  const BinShape bs = pme_grid_make(nfftx, nffty, nfftz, order, unit).b;
+  const int nb = bs.nbins;
   gse_status_t st = h->fft->fft.init(h->ct_dbl, nfftx, nffty, nfftz);
   if (st == GSE_SUCCESS) st = h->counts.ensure(sizeof(int) * (size_t)nb);
+  if (st == GSE_SUCCESS) st = h->bshift.ensure(sizeof(int) * (size_t)nb);
+  if (st == GSE_SUCCESS) st = h->bricks.ensure(8 * (size_t)bs.Lx * bs.Ly * bs.Lz * nb + kBrickPad);
+  // particles as dense as water on a grid of 1 A, and a quarter more: larger
+  // calls allocate once
+  if (st == GSE_SUCCESS) st = h->slots.ensure(pme_slot_bytes(h->ct_dbl, (int)(np / 8), nb));
   if (st == GSE_SUCCESS) st = h->grid64.ensure(8 * np);
   if (st == GSE_SUCCESS) st = h->grid.ensure(tsize(h->ct_dbl) * np);
   if (st == GSE_SUCCESS) st = h->spec.ensure(2 * tsize(h->ct_dbl) * nk);
@@ -1914,8 +1950,9 @@ gse_status_t gse_pme_recip_destroy(gse_pme_recip_t h) {
     delete h->fft;
   }
   for (DevBuf* b : {&h->grid64, &h->grid, &h->spec, &h->prefac, &h->partials, &h->stats, &h->tmp2,
-                    &h->counts, &h->ovf, &h->sorted, &h->bricks, &h->bshift})
+                    &h->counts, &h->slots, &h->bricks, &h->bshift})
     b->release();
+  for (DevBuf& b : h->outgrown) b.release();
   delete h;
   return GSE_SUCCESS;
 }
@@ -1936,22 +1973,19 @@ gse_status_t gse_pme_recip_spread_charge(gse_pme_recip_t h, const void* xyzq, in
   h->n_last = ncoord;
   hipStream_t s = h->stream;
   const PmeGrid a = pme_grid_make(h->X, h->Y, h->Z, h->order, r3);
-  // twice the mean occupancy plus a margin; the rest spreads by itself
-  const int nb = a.b.nbins, cap = (int)((2LL * ncoord / nb + 32 + 15) / 16 * 16);
-  const size_t vol = (size_t)a.b.Lx * a.b.Ly * a.b.Lz;
-  GSECHK(h->bshift.ensure(sizeof(int) * (size_t)nb));
-  GSECHK(h->bricks.ensure(8 * vol * nb + kBrickPad));
-  GSECHK(h->sorted.ensure(4 * tsize(h->ct_dbl) * (size_t)nb * cap));
-  GSECHK(h->ovf.ensure(sizeof(int) * (size_t)std::max(ncoord, 1)));
+  const int nb = a.b.nbins, cap = pme_cap(ncoord, nb);
+  const size_t need = pme_slot_bytes(h->ct_dbl, ncoord, nb);
+  if (need > h->slots.bytes) GSECHK(pme_grow_slots(h, need));
+  int* ovf = (int*)(h->slots.as<char>() + pme_sorted_bytes(h->ct_dbl, ncoord, nb));
   BinStats *st = h->stats.as<BinStats>(), *kept = st + 1;
   const bool dirty = h->dirty;
   h->dirty = true;
   if (dirty) HIPCHK(launch_bin_clear(h->counts.as<int>(), nb, st, s));
   HIPCHK(launch_pme_bin(h->ct_dbl, xyzq, ncoord, a, cap, h->counts.as<int>(), st,
-                        h->ovf.as<int>(), h->sorted.p, s));
+                        ovf, h->slots.p, s));
   HIPCHK(launch_pme_spread(h->ct_dbl, h->order, xyzq, ncoord, a, cap, h->counts.as<int>(), st,
-                           kept, h->ovf.as<int>(), h->sorted.p, h->bricks.p,
-                           h->bshift.as<int>(), h->grid64.as<unsigned long long>(), s));
+                           kept, ovf, h->slots.p, h->bricks.p, h->bshift.as<int>(),
+                           h->grid64.as<unsigned long long>(), s));
   Binning w;
   w.n = ncoord;
   w.stats = kept;

@@ -189,6 +189,27 @@ def test_spme_captured_step_replays_like_the_eager_one():
     assert torch.equal(pm.grid(), ref.grid())
 
 
+def test_spme_first_call_captured_and_outgrown():
+    """A handle's first spread may be captured, with more particles than its
+    buffers were made for, and the graph stays valid after a larger call:
+    replays equal a fresh handle's eager spread bit for bit."""
+    dims, box, n = (24, 18, 33), (24.0, 18.0, 33.0), 4000
+    x = dev(spme_uneven(n, box, 0), F64)
+    more = dev(spme_uneven(30000, box, 3), F64)
+    pm, ref = (api.CudaPMERecip(F64, F64, *dims, 6) for _ in range(2))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        pm.spread_charge(x, n, box)
+    for seed in range(4):
+        x.copy_(dev(spme_uneven(n, box, seed), F64))
+        graph.replay()
+        ref.spread_charge(x, n, box)
+        assert torch.equal(pm.grid(), ref.grid()), seed
+        pm.spread_charge(more, len(more), box)
+        ref.spread_charge(more, len(more), box)
+        assert torch.equal(pm.grid(), ref.grid()), seed
+
+
 def test_spme_bad_arguments():
     with pytest.raises(api._lib.GSEError):
         api.CudaPMERecip(F64, F64, 16, 16, 16, 5)

@@ -228,8 +228,8 @@ __device__ __forceinline__ void pme_contrib(const PmeSplines<ORDER, false>& s, i
 
 // B-spline spread of one bin per workgroup into an int64 brick in LDS
 // (kPmeEdge + ORDER - 1 cells a side), stored whole; k_brick_reduce adds the
-// bricks.  The kOverflowWG workgroups after the bins' add the particles that
-// found their bin full to the int64 grid with global atomics.  Spreading
+// bricks.  The workgroups after the bins' add the particles that found their
+// bin full to the int64 grid with global atomics, `per` at a time.  Spreading
 // every particle that way, 64 atomics of 8 bytes each to memory, took 49 us
 // of the 48,000-charge step at order 4, after 11 us for max |q|; binning,
 // spread and reduce take 5.7 + 10.3 + 8.4 (order 6, 200,001 charges on
@@ -242,7 +242,7 @@ __global__ __launch_bounds__(256) void k_pme_spread(
     const P4<CT>* __restrict__ xyzq, int n, PmeGrid a, int cap, int* __restrict__ counts,
     const BinStats* __restrict__ st, BinStats* __restrict__ st_kept,
     const int* __restrict__ ovf, const P4<CT>* __restrict__ sorted, long long* __restrict__ bricks,
-    int* __restrict__ bshift, unsigned long long* __restrict__ g64) {
+    int* __restrict__ bshift, unsigned long long* __restrict__ g64, int per) {
   constexpr int G = PmeLanes<ORDER>::G, PER = 256 / G;
   constexpr int L = kPmeEdge + ORDER - 1, VOL = L * L * L;
   __shared__ unsigned long long brick[VOL];
@@ -253,10 +253,10 @@ __global__ __launch_bounds__(256) void k_pme_spread(
   const double scale = ldexp(1.0, fixed_exponent(s.qmax_bits, n - s.invalid, 1, 1.0));
   const int bin = blockIdx.x;
   if (bin >= a.b.nbins) {
-    const int w = bin - a.b.nbins;
+    const int w = bin - a.b.nbins, nw = (int)gridDim.x - a.b.nbins;
     if (w == 0 && threadIdx.x == 0) *st_kept = s;
-    for (int k0 = w * kPmeChunk; k0 < s.overflow; k0 += kOverflowWG * kPmeChunk) {
-      const int m = min(kPmeChunk, s.overflow - k0);
+    for (int k0 = w * per; k0 < s.overflow; k0 += nw * per) {
+      const int m = min(per, s.overflow - k0);
       pme_splines<ORDER, false, CT>(sp, a, m, [&](int k) { return xyzq[ovf[k0 + k]]; });
       __syncthreads();
       for (int k = threadIdx.x / G; k < m; k += PER)
@@ -497,14 +497,29 @@ hipError_t launch_pme_bin(bool dbl, const void* xyzq, int n, const PmeGrid& a, i
   return hipGetLastError();
 }
 
+// particles per workgroup: whole chunks once they still make four workgroups
+// per CU
+template <int ORDER>
+static int pme_per_wg(int n) {
+  constexpr int PER = 256 / PmeLanes<ORDER>::G;
+  return std::min(kPmeChunk, std::max(1, n / (1024 * PER)) * PER);
+}
+
 template <int ORDER, typename CT>
 static void pme_spread_t(const void* xyzq, int n, const PmeGrid& a, int cap, int* counts,
                          const BinStats* st, BinStats* st_kept, const int* ovf,
                          const void* sorted, void* bricks, int* bshift, unsigned long long* g64,
                          hipStream_t s) {
-  k_pme_spread<ORDER, CT><<<a.b.nbins + kOverflowWG, 256, 0, s>>>(
+  // Overflow workgroups for all the particles (up to eight per CU): a box
+  // filled in a tenth of its volume has most of them on the overflow list.
+  // The call then took 205 us at order 4 (48,000 charges, 80^3) and 699 at
+  // order 8 with eight such workgroups, 57 and
+  // 208 now; without overflow it takes 22 and 42.
+  const int per = pme_per_wg<ORDER>(n);
+  const int ovf_wg = std::max(1, std::min(2048, (n + per - 1) / per));
+  k_pme_spread<ORDER, CT><<<a.b.nbins + ovf_wg, 256, 0, s>>>(
       (const P4<CT>*)xyzq, n, a, cap, counts, st, st_kept, ovf, (const P4<CT>*)sorted,
-      (long long*)bricks, bshift, g64);
+      (long long*)bricks, bshift, g64, per);
 }
 
 hipError_t launch_pme_spread(bool dbl, int order, const void* xyzq, int n, const PmeGrid& a,
@@ -562,9 +577,7 @@ template <int ORDER, typename CT>
 static void pme_gather_o(bool at_dbl, const void* xyzq, int n, int X, int Y, int Z,
                          const double* r, double ccelec, double sign, const void* Qc, void* ox,
                          void* oy, void* oz, hipStream_t s) {
-  constexpr int PER = 256 / PmeLanes<ORDER>::G;
-  // whole chunks once they still make four workgroups per CU
-  const int per = std::min(kPmeChunk, std::max(1, n / (1024 * PER)) * PER);
+  const int per = pme_per_wg<ORDER>(n);
   const unsigned grid = (unsigned)((n + per - 1) / per);
   const PmeGrid g = pme_grid_make(X, Y, Z, ORDER, r);
   if (at_dbl)

@@ -210,6 +210,23 @@ def test_spme_first_call_captured_and_outgrown():
         assert torch.equal(pm.grid(), ref.grid()), seed
 
 
+def test_spme_one_handle_many_sizes():
+    """One handle over calls of very different numbers of particles: more on
+    the overflow list than its workgroups take in one round (2048 of 64), none
+    at all, rejected ones before good ones.  Grids against the oracle."""
+    dims, box = (16, 16, 16), (16.0, 16.0, 16.0)
+    rng = np.random.default_rng(2)
+    pm = api.CudaPMERecip(F64, F64, *dims, 4)
+    for n, spread, bad in ((200000, 0.4, 0), (7, 1.0, 3), (0, 1.0, 0), (5000, 0.3, 40), (3000, 1.0, 0)):
+        x = np.empty((n, 4))
+        x[:, :3] = rng.random((n, 3)) * box * spread
+        x[:, 3] = rng.standard_normal(n)
+        x[:bad, rng.integers(4)] = np.inf
+        pm.spread_charge(dev(x), n, box)
+        q = orc.pme_spread(dims, 4, x[bad:], box) if n else np.zeros(dims[::-1])
+        assert rel(host(pm.grid()).ravel(), np.asarray(q).ravel()) <= TOL, n
+
+
 def test_spme_bad_arguments():
     with pytest.raises(api._lib.GSEError):
         api.CudaPMERecip(F64, F64, 16, 16, 16, 5)

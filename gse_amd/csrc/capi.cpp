@@ -1852,7 +1852,9 @@ gse_status_t pme_recip3(const double* recip, double* r3) {
 
 // slots per bin for n particles: twice the mean occupancy plus a margin; the
 // rest spreads by itself
-int pme_cap(int n, int nb) { return (int)((2LL * n / nb + 32 + 15) / 16 * 16); }
+int pme_cap(int n, int nb) {
+  return (int)std::min((2LL * n / nb + 32 + 15) / 16 * 16, 1LL << 30);
+}
 size_t pme_sorted_bytes(bool dbl, int n, int nb) {
   return 4 * tsize(dbl) * (size_t)nb * pme_cap(n, nb);
 }
@@ -1911,10 +1913,6 @@ gse_status_t gse_pme_recip_create(gse_pme_recip_t* out, gse_dtype_t at, gse_dtyp
   gse_status_t st = h->fft->fft.init(h->ct_dbl, nfftx, nffty, nfftz);
   if (st == GSE_SUCCESS) st = h->counts.ensure(sizeof(int) * (size_t)nb);
   if (st == GSE_SUCCESS) st = h->bshift.ensure(sizeof(int) * (size_t)nb);
-  if (st == GSE_SUCCESS) st = h->bricks.ensure(8 * (size_t)bs.Lx * bs.Ly * bs.Lz * nb + kBrickPad);
-  // particles as dense as water on a grid of 1 A, and a quarter more: larger
-  // calls allocate once
-  if (st == GSE_SUCCESS) st = h->slots.ensure(pme_slot_bytes(h->ct_dbl, (int)(np / 8), nb));
   if (st == GSE_SUCCESS) st = h->grid64.ensure(8 * np);
   if (st == GSE_SUCCESS) st = h->grid.ensure(tsize(h->ct_dbl) * np);
   if (st == GSE_SUCCESS) st = h->spec.ensure(2 * tsize(h->ct_dbl) * nk);
@@ -1922,6 +1920,16 @@ gse_status_t gse_pme_recip_create(gse_pme_recip_t* out, gse_dtype_t at, gse_dtyp
   if (st == GSE_SUCCESS) st = h->partials.ensure(sizeof(double) * 7 * kPmeSumBlocks);
   if (st == GSE_SUCCESS) st = h->stats.ensure(2 * sizeof(BinStats));
   if (st == GSE_SUCCESS) st = h->tmp2.ensure(sizeof(double) * (kRedBlocks * 2 + 2));
+  // bricks (21 bytes a grid cell at order 4, 53 at order 8), and slots for
+  // particles as dense as water on a grid of 1 A and a quarter more (larger
+  // calls allocate once); where memory does not allow them the spread does
+  // without
+  if (st == GSE_SUCCESS &&
+      (h->bricks.ensure(8 * (size_t)bs.Lx * bs.Ly * bs.Lz * nb + kBrickPad) != GSE_SUCCESS ||
+       h->slots.ensure(pme_slot_bytes(h->ct_dbl, (int)(np / 8), nb)) != GSE_SUCCESS)) {
+    h->bricks.release();
+    (void)hipGetLastError();
+  }
   if (st == GSE_SUCCESS) {
     std::vector<double> pf((size_t)nfftx + nffty + nfftz);
     pme_moduli(order, nfftx, pf.data());
@@ -1972,24 +1980,39 @@ gse_status_t gse_pme_recip_spread_charge(gse_pme_recip_t h, const void* xyzq, in
   std::memcpy(h->recip3, r3, sizeof(r3));
   h->n_last = ncoord;
   hipStream_t s = h->stream;
-  const PmeGrid a = pme_grid_make(h->X, h->Y, h->Z, h->order, r3);
+  PmeGrid a = pme_grid_make(h->X, h->Y, h->Z, h->order, r3);
   const int nb = a.b.nbins, cap = pme_cap(ncoord, nb);
   const size_t need = pme_slot_bytes(h->ct_dbl, ncoord, nb);
-  if (need > h->slots.bytes) GSECHK(pme_grow_slots(h, need));
-  int* ovf = (int*)(h->slots.as<char>() + pme_sorted_bytes(h->ct_dbl, ncoord, nb));
+  bool bins = h->bricks.p && g_tuning.spread_flush;
+  if (bins && need > h->slots.bytes && pme_grow_slots(h, need) != GSE_SUCCESS) {
+    bins = false;
+    (void)hipGetLastError();
+  }
   BinStats *st = h->stats.as<BinStats>(), *kept = st + 1;
   const bool dirty = h->dirty;
   h->dirty = true;
   if (dirty) HIPCHK(launch_bin_clear(h->counts.as<int>(), nb, st, s));
+  Binning w;
+  w.n = ncoord;
+  w.stats = kept;
+  w.pref_bound = 1.0;
+  if (!bins) {  // every particle with global atomics
+    HIPCHK(launch_pme_bin(h->ct_dbl, xyzq, ncoord, a, 0, nullptr, st, nullptr, nullptr, s));
+    a.b.nbins = 0;
+    HIPCHK(launch_pme_spread(h->ct_dbl, h->order, xyzq, ncoord, a, 0, nullptr, st, kept, nullptr,
+                             nullptr, nullptr, nullptr, h->grid64.as<unsigned long long>(), s));
+    HIPCHK(launch_fixed_to_grid(h->ct_dbl, h->grid64.as<unsigned long long>(), h->grid.p,
+                                (size_t)h->X * h->Y * h->Z, w, true, s));
+    HIPCHK(launch_bin_clear(h->counts.as<int>(), nb, st, s));
+    h->dirty = dirty;
+    return GSE_SUCCESS;
+  }
+  int* ovf = (int*)(h->slots.as<char>() + pme_sorted_bytes(h->ct_dbl, ncoord, nb));
   HIPCHK(launch_pme_bin(h->ct_dbl, xyzq, ncoord, a, cap, h->counts.as<int>(), st,
                         ovf, h->slots.p, s));
   HIPCHK(launch_pme_spread(h->ct_dbl, h->order, xyzq, ncoord, a, cap, h->counts.as<int>(), st,
                            kept, ovf, h->slots.p, h->bricks.p, h->bshift.as<int>(),
                            h->grid64.as<unsigned long long>(), s));
-  Binning w;
-  w.n = ncoord;
-  w.stats = kept;
-  w.pref_bound = 1.0;
   w.bricks = h->bricks.p;
   w.bshift = h->bshift.as<int>();
   const Geom g = make_geom(h->X, h->Y, h->Z, 1.0, 1.0, 1.0, 1.0);

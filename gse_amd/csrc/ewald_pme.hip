@@ -104,7 +104,8 @@ struct PmeLanes {
 // support, with max |q| and the rejected count of the call.  Slots are
 // claimed as the GSE binning claims them: one global atomic per workgroup
 // and touched bin, ranks within it from LDS (above kPmeAggBins bins, one per
-// particle: a workgroup's particles then touch most bins once).
+// particle: a workgroup's particles then touch most bins once).  Without
+// counts, the statistics only.
 constexpr int kPmeEdge = 8, kPmeAggBins = 16384;
 template <typename CT>
 __global__ __launch_bounds__(1024) void k_pme_bin(const P4<CT>* __restrict__ xyzq, int n,
@@ -149,7 +150,7 @@ __global__ __launch_bounds__(1024) void k_pme_bin(const P4<CT>* __restrict__ xyz
       if (c > 0) pme_hist[j] = atomicAdd(&counts[j], c);
     }
   __syncthreads();
-  if (bin >= 0) {
+  if (bin >= 0 && counts) {
     const int slot = agg ? pme_hist[bin] + rank : atomicAdd(&counts[bin], 1);
     if (slot < cap)
       sorted[(size_t)bin * cap + slot] = r;
@@ -229,7 +230,8 @@ __device__ __forceinline__ void pme_contrib(const PmeSplines<ORDER, false>& s, i
 // B-spline spread of one bin per workgroup into an int64 brick in LDS
 // (kPmeEdge + ORDER - 1 cells a side), stored whole; k_brick_reduce adds the
 // bricks.  The workgroups after the bins' add the particles that found their
-// bin full to the int64 grid with global atomics, `per` at a time.  Spreading
+// bin full to the int64 grid with global atomics, `per` at a time (without an
+// overflow list and bins, all the particles).  Spreading
 // every particle that way, 64 atomics of 8 bytes each to memory, took 49 us
 // of the 48,000-charge step at order 4, after 11 us for max |q|; binning,
 // spread and reduce take 5.7 + 10.3 + 8.4 (order 6, 200,001 charges on
@@ -255,12 +257,14 @@ __global__ __launch_bounds__(256) void k_pme_spread(
   if (bin >= a.b.nbins) {
     const int w = bin - a.b.nbins, nw = (int)gridDim.x - a.b.nbins;
     if (w == 0 && threadIdx.x == 0) *st_kept = s;
-    for (int k0 = w * per; k0 < s.overflow; k0 += nw * per) {
-      const int m = min(per, s.overflow - k0);
-      pme_splines<ORDER, false, CT>(sp, a, m, [&](int k) { return xyzq[ovf[k0 + k]]; });
+    const int novf = ovf ? s.overflow : n;
+    for (int k0 = w * per; k0 < novf; k0 += nw * per) {
+      const int m = min(per, novf - k0);
+      pme_splines<ORDER, false, CT>(sp, a, m,
+                                    [&](int k) { return xyzq[ovf ? ovf[k0 + k] : k0 + k]; });
       __syncthreads();
       for (int k = threadIdx.x / G; k < m; k += PER)
-        if (live)
+        if (live && sp.q[k] == sp.q[k])
           pme_contrib<ORDER>(sp, k, scale, ax, ay, [&](int x, int y, int z, long long v) {
             x = x >= a.X ? x - a.X : x;
             y = y >= a.Y ? y - a.Y : y;
@@ -485,7 +489,7 @@ PmeGrid pme_grid_make(int X, int Y, int Z, int order, const double* r) {
 hipError_t launch_pme_bin(bool dbl, const void* xyzq, int n, const PmeGrid& a, int cap,
                           int* counts, BinStats* st, int* ovf, void* sorted, hipStream_t s) {
   if (n <= 0) return hipSuccess;
-  const int agg = a.b.nbins <= kPmeAggBins ? 1 : 0;
+  const int agg = counts && a.b.nbins <= kPmeAggBins ? 1 : 0;
   const unsigned g = (unsigned)((n + 1023) / 1024);
   const size_t lds = agg ? sizeof(int) * (size_t)a.b.nbins : 0;
   if (dbl)

@@ -464,11 +464,12 @@ struct PmeGrid {
 };
 PmeGrid pme_grid_make(int X, int Y, int Z, int order, const double* recip3);
 // bins: cap slots each in sorted [nbins * cap], counts [nbins] and st zero on
-// entry; the rest into ovf [n]
+// entry; the rest into ovf [n].  counts NULL: the statistics only
 hipError_t launch_pme_bin(bool dbl, const void* xyzq, int n, const PmeGrid& a, int cap,
                           int* counts, BinStats* st, int* ovf, void* sorted, hipStream_t s);
 // bricks [nbins][L^3] int64 and bshift [nbins] for launch_brick_reduce_list,
-// overflow particles into g64; clears counts, copies st to st_kept
+// overflow particles into g64; clears counts, copies st to st_kept.  ovf NULL
+// and no bins (a.b.nbins 0): every particle into g64
 hipError_t launch_pme_spread(bool dbl, int order, const void* xyzq, int n, const PmeGrid& a,
                              int cap, int* counts, const BinStats* st, BinStats* st_kept,
                              const int* ovf, const void* sorted, void* bricks, int* bshift,

@@ -77,7 +77,9 @@ GSE_API gse_status_t gse_set_tiling(int bin_edge, int lds_budget_bytes);
  *   spread_lds32  FP32 grids: 32-bit accumulators, per-bin scale (0/1, 1)
  *   spread_cols   column-owner register spread (0/1, 0); 0 = LDS-atomic brick
  *   spread_flush  1: each bin stores its brick and one pass sums the bricks
- *                 covering each grid point; 0: bricks added with atomics (0/1, 1)
+ *                 covering each grid point; 0: bricks added with atomics (0/1, 1).
+ *                 SPME: 0 spreads every particle with atomics, as it does by
+ *                 itself where memory is short for the bricks
  *   reduce_tile   that sum by one workgroup per 8^3 bin where the grid allows (0/1, 1)
  *   reduce_nt     brick loads of that FP32 sum: 0 ordinary, 1 non-temporal (0/1, 0)
  *   reduce_tile2  that sum over 64-bit bricks with two x points per thread (0/1, 1)

@@ -227,6 +227,26 @@ def test_spme_one_handle_many_sizes():
         assert rel(host(pm.grid()).ravel(), np.asarray(q).ravel()) <= TOL, n
 
 
+@pytest.mark.parametrize("dt,order", [(F32, 4), (F64, 6), (F32, 8)])
+def test_spme_without_bricks(dt, order):
+    """The spread without bins and bricks (taken where memory is short for
+    them): the same integers, so the same grid, with rejected particles, and
+    neither route leaves anything behind for the other."""
+    dims, box, n = (24, 18, 33), (24.0, 18.0, 33.0), 2500
+    pm, ref = (api.CudaPMERecip(dt, dt, *dims, order) for _ in range(2))
+    try:
+        for seed in range(4):
+            x = dev(spme_uneven(n, box, seed), dt)
+            ref.spread_charge(x, n, box)
+            for flush in (0, 1, 0):
+                api.set_tuning(spread_flush=flush)
+                pm.spread_charge(x, n, box)
+                assert torch.equal(pm.grid(), ref.grid()), (seed, flush)
+            api.set_tuning(spread_flush=1)
+    finally:
+        api.set_tuning(spread_flush=1)
+
+
 def test_spme_bad_arguments():
     with pytest.raises(api._lib.GSEError):
         api.CudaPMERecip(F64, F64, 16, 16, 16, 5)

@@ -1073,7 +1073,7 @@ template <int WAVES>
 __device__ __forceinline__ void mma_tables(const SpreadArgs& a, MmaLds& m, int c0, int kc, int cnt,
                                            const V4<float>* __restrict__ slots,
                                            const int* __restrict__ loc,
-                                           const V4<float>* __restrict__ xyzq, float qscale) {
+                                           const V4<float>* __restrict__ xyzq, int eq) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nks = (kc + 63) >> 6;
@@ -1118,8 +1118,9 @@ __device__ __forceinline__ void mma_tables(const SpreadArgs& a, MmaLds& m, int c
       const int c = (int)round(xv * ih) - (kMmaNZC - 1) / 2;
       const double d0 = sub_rn(mul_rn((double)c, h), xv);
       const int first = axis == 0 ? o & 255 : axis == 1 ? o >> 8 & 255 : o >> 16;
+      // ldexp: the scale itself may lie outside the range of FP32
       const float scale =
-          axis == 0 ? fabsf(p.w) * qscale : axis == 1 ? 1.0f : copysignf(kMmaSpanB, p.w);
+          axis == 0 ? ldexpf(fabsf(p.w), eq) : axis == 1 ? 1.0f : copysignf(kMmaSpanB, p.w);
       for (int j = lo; j < hi; j++) {
         const float tc = (float)add_rn(d0, mul_rn((double)j, h));
         const float w = scale * gexp(mul_rn(mul_rn(-tc, tc), (float)a.inv2s2));
@@ -1177,7 +1178,7 @@ __device__ __forceinline__ void mma_bin(const SpreadArgs& a, MmaLds& m, int bin,
     mma_giant_bin<WAVES>(a, slots, cnt, eg, shift, grid64);
     return;
   }
-  // the total T = sum A B is q wx wy wz at the scale qscale kMmaSpanB and goes
+  // the total T = sum A B is q wx wy wz at the scale 2^eq kMmaSpanB and goes
   // to the brick's q pref wx wy wz 2^(eg - shift), rounded once
   union {
     unsigned long long u;
@@ -1187,7 +1188,6 @@ __device__ __forceinline__ void mma_bin(const SpreadArgs& a, MmaLds& m, int bin,
   int eq = 0;
   const double qm = frexp(qv.d, &eq);  // in [1/2, 1)
   eq = qm * 8388608.0 < (double)kMmaSpan ? 23 - eq : 22 - eq;
-  const float qscale = qv.d > 0.0 ? (float)ldexp(1.0, eq) : 0.0f;
   const double fct = qv.d > 0.0 ? ldexp(a.pref / (double)kMmaSpanB, eg - shift - eq) : 0.0;
   const double f1 = fct * 256.0, f2 = fct * 65536.0, f3 = fct * 16777216.0;
   if (call > cnt) {  // the bin's overflow particles, from the overflow list
@@ -1201,7 +1201,7 @@ __device__ __forceinline__ void mma_bin(const SpreadArgs& a, MmaLds& m, int bin,
   }
   const bool once = call <= kMmaK;
   if (once) {
-    mma_tables<WAVES>(a, m, 0, call, cnt, slots, loc, xyzq, qscale);
+    mma_tables<WAVES>(a, m, 0, call, cnt, slots, loc, xyzq, eq);
     __syncthreads();
   }
   // exact class sums -> brick values at 2^(eg - shift): they convert to FP64
@@ -1237,7 +1237,7 @@ __device__ __forceinline__ void mma_bin(const SpreadArgs& a, MmaLds& m, int bin,
       const int kc = min(kMmaK, call - c0);
       if (!once) {  // more particles than the tables hold: rebuilt per row tile
         __syncthreads();
-        mma_tables<WAVES>(a, m, c0, kc, cnt, slots, loc, xyzq, qscale);
+        mma_tables<WAVES>(a, m, c0, kc, cnt, slots, loc, xyzq, eq);
         __syncthreads();
       }
       for (int ks = 0; mine && 64 * ks < kc; ks++) {

@@ -140,6 +140,19 @@ def test_mma_spread_bin_counts(extra):
     assert err <= bound
 
 
+@pytest.mark.parametrize("scale", [1e-35, 1e-33, 1e-31, 1e30, 1e35])
+def test_mma_spread_charge_scale(scale):
+    """Charges of any size: the factors are scaled by a power of two, which
+    for charges below 2^-105 lies beyond FP32."""
+    xyzq = systems.water_box(1000, 31.0, seed=3)
+    xyzq[:, 3] *= scale
+    p = orc.Params(32, 31.0, 2.12)
+    r1, lay = spread32(xyzq, p, 2)
+    assert lay["spread"] == "mma"
+    ref = orc.spread(p.dims, p.sigma1, p.rcut1, xyzq.astype(np.float32).astype(np.float64), p.box)
+    assert rel(host(r1), ref) <= 2e-6
+
+
 def test_mma_spread_giant_bin_takes_the_per_contribution_path():
     """A bin with more than 500 particles is spread per contribution
     (int32 class sums would no longer be exact): with every particle in that

@@ -1074,17 +1074,21 @@ __device__ __forceinline__ void mma_tables(const SpreadArgs& a, MmaLds& m, int c
                                            const V4<float>* __restrict__ slots,
                                            const int* __restrict__ loc,
                                            const V4<float>* __restrict__ xyzq, int eq) {
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int tid = threadIdx.x;
+  // opaque, so that no address is computed before a loop over several builds:
+  // held across it they would spill 20 registers
+  asm volatile("" : "+v"(tid));
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nks = (kc + 63) >> 6;
   const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
   for (int ks = 0; ks < nks; ks++) {
-    for (int e = threadIdx.x; e < kMmaL * 16; e += (64 * WAVES)) {
+    for (int e = tid; e < kMmaL * 16; e += (64 * WAVES)) {
       const int at = (e >> 4) * kMmaPitch + 64 * ks + 4 * (e & 15);
       *(float4*)&m.x[at] = zero;
       *(float4*)&m.y[at] = zero;
     }
-    for (int e = threadIdx.x; e < 32 * 4; e += (64 * WAVES)) {
+    for (int e = tid; e < 32 * 4; e += (64 * WAVES)) {
       *(float4*)&m.b[0][ks][0][16 * e] = zero;
       *(float4*)&m.b[1][ks][0][16 * e] = zero;
       *(float4*)&m.b[2][ks][0][16 * e] = zero;
@@ -1199,11 +1203,6 @@ __device__ __forceinline__ void mma_bin(const SpreadArgs& a, MmaLds& m, int bin,
     }
     __syncthreads();
   }
-  const bool once = call <= kMmaK;
-  if (once) {
-    mma_tables<WAVES>(a, m, 0, call, cnt, slots, loc, xyzq, eq);
-    __syncthreads();
-  }
   // exact class sums -> brick values at 2^(eg - shift): they convert to FP64
   // exactly, the weighted sum is formed in a fixed order and rounded once (the
   // same operations for any order of the particles)
@@ -1225,63 +1224,89 @@ __device__ __forceinline__ void mma_bin(const SpreadArgs& a, MmaLds& m, int bin,
 #pragma unroll
   for (int c = 0; c < 4; c++) top[c] = mma_v4i{0, 0, 0, 0};
   constexpr int kRounds = (kMmaTiles + WAVES - 1) / WAVES;
-  for (int t = 0; t < kRounds; t++) {
-    const int tile = wave + WAVES * t, row = 16 * tile + l16;
-    const bool mine = tile < kMmaTiles;  // wave-uniform
-    const int y = row / kMmaL, x = row - y * kMmaL;
-    const int ctop = (l16 >> 2) == (t & 3) ? 16 + (l16 & 3) : kMmaL;
-    mma_v4i acc[4];
+  // The wave's row tiles t0 .. t0 + U - 1.  U = 1 with the tables of all the
+  // particles in place.  U = 2 where the tables hold only a part of them and are
+  // built anew for each part: they then serve two tiles of every wave.  (With
+  // tables per tile, one bin past 128 made the spread of 80^3 wait 40 us: 120 a
+  // bin in 60 % of the box took 94 us, 73 now, the LDS path 85.  Four tiles at
+  // once spill: 160^3 evenly filled 227 -> 245 us.)
+  auto rounds = [&](auto width, int t0) {
+    constexpr int U = decltype(width)::value;
+    mma_v4i acc[U][4];
 #pragma unroll
-    for (int c = 0; c < 4; c++) acc[c] = mma_v4i{0, 0, 0, 0};
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int c = 0; c < 4; c++) acc[u][c] = mma_v4i{0, 0, 0, 0};
     for (int c0 = 0; c0 < call; c0 += kMmaK) {
       const int kc = min(kMmaK, call - c0);
-      if (!once) {  // more particles than the tables hold: rebuilt per row tile
+      if (U > 1) {
         __syncthreads();
         mma_tables<WAVES>(a, m, c0, kc, cnt, slots, loc, xyzq, eq);
         __syncthreads();
       }
-      for (int ks = 0; mine && 64 * ks < kc; ks++) {
-        const float4* px = (const float4*)&m.x[x * kMmaPitch + 64 * ks + 16 * grp];
-        const float4* py = (const float4*)&m.y[y * kMmaPitch + 64 * ks + 16 * grp];
-        mma_v4i a0, a1, a2, a3;
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-          int l0, l1, l2, l3;
-          mma_limbs4(px[q], py[q], l0, l1, l2, l3);
-          a0[q] = l0;
-          a1[q] = l1;
-          a2[q] = l2;
-          a3[q] = l3;
+      for (int u = 0; u < U; u++) {
+        const int t = t0 + u, tile = wave + WAVES * t, row = 16 * tile + l16;
+        const bool mine = tile < kMmaTiles;  // wave-uniform
+        const int y = row / kMmaL, x = row - y * kMmaL;
+        const int ctop = (l16 >> 2) == (t & 3) ? 16 + (l16 & 3) : kMmaL;
+        for (int ks = 0; mine && 64 * ks < kc; ks++) {
+          const float4* px = (const float4*)&m.x[x * kMmaPitch + 64 * ks + 16 * grp];
+          const float4* py = (const float4*)&m.y[y * kMmaPitch + 64 * ks + 16 * grp];
+          mma_v4i a0, a1, a2, a3;
+#pragma unroll
+          for (int q = 0; q < 4; q++) {
+            int l0, l1, l2, l3;
+            mma_limbs4(px[q], py[q], l0, l1, l2, l3);
+            a0[q] = l0;
+            a1[q] = l1;
+            a2[q] = l2;
+            a3[q] = l3;
+            if (U > 1) __builtin_amdgcn_sched_barrier(0);
+          }
+          auto step = [&](mma_v4i(&d)[4], int col) {
+            const mma_v4i b0 = *(const mma_v4i*)&m.b[0][ks][col][16 * grp];
+            const mma_v4i b1 = *(const mma_v4i*)&m.b[1][ks][col][16 * grp];
+            const mma_v4i b2 = *(const mma_v4i*)&m.b[2][ks][col][16 * grp];
+            const mma_v4i b3 = *(const mma_v4i*)&m.b[3][ks][col][16 * grp];
+            // limb classes of weight 2^8 (a0 b1 + a1 b0 + a2 b3 + a3 b2), 2^16
+            // (a0 b2 + a1 b1 + a2 b0), 2^24 (a1 b2 + a2 b1) and 2^32 (a2 b2)
+            d[0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, b1, d[0], 0, 0, 0);
+            d[1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, b2, d[1], 0, 0, 0);
+            d[2] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, b2, d[2], 0, 0, 0);
+            d[3] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a2, b2, d[3], 0, 0, 0);
+            d[0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, b0, d[0], 0, 0, 0);
+            d[1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, b1, d[1], 0, 0, 0);
+            d[2] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a2, b1, d[2], 0, 0, 0);
+            d[0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a2, b3, d[0], 0, 0, 0);
+            d[1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a2, b0, d[1], 0, 0, 0);
+            d[0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a3, b2, d[0], 0, 0, 0);
+          };
+          step(acc[u], l16);
+          if (U > 1) __builtin_amdgcn_sched_barrier(0);
+          step(top, ctop);
+          if (U > 1) __builtin_amdgcn_sched_barrier(0);
         }
-        auto step = [&](mma_v4i(&d)[4], int col) {
-          const mma_v4i b0 = *(const mma_v4i*)&m.b[0][ks][col][16 * grp];
-          const mma_v4i b1 = *(const mma_v4i*)&m.b[1][ks][col][16 * grp];
-          const mma_v4i b2 = *(const mma_v4i*)&m.b[2][ks][col][16 * grp];
-          const mma_v4i b3 = *(const mma_v4i*)&m.b[3][ks][col][16 * grp];
-          // limb classes of weight 2^8 (a0 b1 + a1 b0 + a2 b3 + a3 b2), 2^16
-          // (a0 b2 + a1 b1 + a2 b0), 2^24 (a1 b2 + a2 b1) and 2^32 (a2 b2)
-          d[0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, b1, d[0], 0, 0, 0);
-          d[1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, b2, d[1], 0, 0, 0);
-          d[2] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, b2, d[2], 0, 0, 0);
-          d[3] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a2, b2, d[3], 0, 0, 0);
-          d[0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, b0, d[0], 0, 0, 0);
-          d[1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, b1, d[1], 0, 0, 0);
-          d[2] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a2, b1, d[2], 0, 0, 0);
-          d[0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a2, b3, d[0], 0, 0, 0);
-          d[1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a2, b0, d[1], 0, 0, 0);
-          d[0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a3, b2, d[0], 0, 0, 0);
-        };
-        step(acc, l16);
-        step(top, ctop);
       }
     }
-    if (mine) put(acc, 16 * tile + 4 * grp + kMmaLXY * l16);
-    if ((t & 3) == 3 || t == kRounds - 1) {
-      const int q = wave + WAVES * ((t & ~3) + (l16 >> 2));  // the tile of this column
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int tile = wave + WAVES * (t0 + u);
+      if (tile < kMmaTiles) put(acc[u], 16 * tile + 4 * grp + kMmaLXY * l16);
+    }
+    if (((t0 + U) & 3) == 0 || t0 + U >= kRounds) {
+      const int q = wave + WAVES * ((t0 & ~3) + (l16 >> 2));  // the tile of this column
       if (q < kMmaTiles) put(top, 16 * q + 4 * grp + kMmaLXY * (16 + (l16 & 3)));
 #pragma unroll
       for (int c = 0; c < 4; c++) top[c] = mma_v4i{0, 0, 0, 0};
     }
+  };
+  if (call <= kMmaK) {
+    mma_tables<WAVES>(a, m, 0, call, cnt, slots, loc, xyzq, eq);
+    __syncthreads();
+    for (int t = 0; t < kRounds; t++) rounds(std::integral_constant<int, 1>{}, t);
+  } else {
+    for (int t = 0; t < kRounds; t += 2) rounds(std::integral_constant<int, 2>{}, t);
   }
 }
 
@@ -1337,12 +1362,16 @@ bool spread_mma_ok(bool dbl, const Geom& g, const BinShape& b, bool normalize, b
   if (b.Lx != kMmaL || b.Ly != kMmaL || b.Lz != kMmaL) return false;
   // Automatic choice by the mean number of charges per bin.  A brick costs the
   // matrix path the same from 1 to 64 charges and little more to 128, the LDS
-  // path in proportion to them; a bin past 128 rebuilds the tables for every
-  // row tile (30 us for the first, with a whole launch waiting for it).
+  // path in proportion to them; a bin past 128 builds the tables several times,
+  // and the launch waits for it.
   // Measured, LDS / matrix us: 80^3 with 18 a bin 22.1 / 24.7, 24 25.4 / 25.0,
   // 36 29.7 / 25.4, 48 34.8 / 26.0, 72 44.7 / 29.1, 96 54.0 / 61.0; 160^3 with
   // 18 104 / 118, 24 115 / 118, 36 143 / 118, 72 242 / 160; 40^3 with 18 13.8 /
-  // 12.9, 72 23.8 / 15.5, 96 26.9 / 30.7.
+  // 12.9, 72 23.8 / 15.5, 96 26.9 / 30.7.  The mean also decides for boxes filled
+  // in part, where it says less: the whole call at 80^3 with half the box
+  // empty takes 71.4 / 46.6 us at 96 charges in a filled bin and 95.2 / 81.3 at
+  // 144; 160^3 561 / 470 at 144; with more than two thirds empty the LDS path's
+  // overflow costs over 1 ms.
   const int knob = tuning().spread_mma;
   return knob == 1 || (knob == 2 && n >= 24LL * b.nbins && n <= 72LL * b.nbins);
 }

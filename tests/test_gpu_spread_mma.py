@@ -140,6 +140,32 @@ def test_mma_spread_bin_counts(extra):
     assert err <= bound
 
 
+@pytest.mark.parametrize("dims", [(66, 72, 70), (40, 40, 40)], ids=["4waves", "8waves"])
+def test_mma_spread_bins_past_the_tables(dims):
+    """Bins of 100 to 500 charges side by side (tables of 128, built anew for
+    each part of a bin and two row tiles a wave), with four and with eight waves
+    a bin: the LDS kernel's grid within FP32 accuracy, and the same bits in any
+    order of the particles."""
+    rng = np.random.default_rng(dims[0])
+    box = tuple(float(m) for m in dims)
+    parts = []
+    for i, n in enumerate((100, 128, 129, 192, 256, 257, 384, 385, 499)):
+        a = rng.random((n, 4)) * np.array([6.0, 6.0, 6.0, 1.0])
+        a[:, :3] += 8.0 * np.array([i % 3, i // 3, i % 2]) + 7.0  # cube origins in one bin
+        parts.append(a)
+    xyzq = np.concatenate(parts + [rng.random((1000, 4)) * np.array([*box, 1.0])])
+    xyzq[:, 3] = rng.choice([-0.834, 0.417], len(xyzq))
+    p = orc.Params(dims, box, 2.12)
+    r1, lay = spread32(xyzq, p, True)
+    r0, _ = spread32(xyzq, p, False)
+    assert lay["spread"] == "mma"
+    assert rel(host(r1), host(r0)) <= 2e-6
+    ref = orc.spread(p.dims, p.sigma1, p.rcut1, xyzq.astype(np.float32).astype(np.float64), p.box)
+    assert rel(host(r1), ref) <= 2e-6
+    r2, _ = spread32(xyzq[rng.permutation(len(xyzq))], p, True)
+    assert torch.equal(r1, r2)
+
+
 @pytest.mark.parametrize("scale", [1e-35, 1e-33, 1e-31, 1e30, 1e35])
 def test_mma_spread_charge_scale(scale):
     """Charges of any size: the factors are scaled by a power of two, which

@@ -834,7 +834,7 @@ struct gse_gseu_s {
   struct Chunk {
     UTaps t[2];          // y and z taps of the chunk's terms
     size_t xtap = 0;     // first of its x taps in `taps`
-    int Rx = 0;
+    int Rx = 0, R[kUTerms][3] = {};
     size_t at[2][kUTerms] = {};  // first y and z tap of each term in `taps`
   };
   std::vector<Chunk> chunks;
@@ -883,7 +883,10 @@ gse_status_t gseu_terms(gse_gseu_s* h, double sigma, double ls1) {
       }
     }
     gse_gseu_s::Chunk ch;
-    for (int k = 0; k < nt; k++) ch.Rx = std::max(ch.Rx, R[k][0]);
+    for (int k = 0; k < nt; k++) {
+      ch.Rx = std::max(ch.Rx, R[k][0]);
+      std::copy(R[k], R[k] + 3, ch.R[k]);
+    }
     ch.xtap = all.size();
     all.resize(ch.xtap + (size_t)(2 * ch.Rx + 1) * kUTerms, 0.0);
     for (int k = 0; k < nt; k++)
@@ -2459,6 +2462,11 @@ gse_status_t gse_gseu_spread_charge1(gse_gseu_t h, int n, const void* xyzq) {
 gse_status_t gse_gseu_solve_poisson(gse_gseu_t h) {
   if (!h) return fail(GSE_ERROR_INVALID_VALUE, "handle is NULL");
   gse_gsek_s* c = h->core;
+  for (const auto& k : h->chunks)  // the limits of one convolution per term
+    for (int j = 0; j < k.t[0].nterm; j++)
+      for (int a = 0; a < 3; a++)
+        if (!conv_pass_ok(c->ct_dbl, a, c->X, c->Y, c->Z, k.R[j][a]))
+          HIPCHK(hipErrorInvalidConfiguration);
   // phiM = rhoG_{N-1} + ... + rhoG_0 (CpuGSEu.cpp:60-66)
   bool add = false;
   for (const auto& k : h->chunks) {

@@ -1312,6 +1312,19 @@ hipError_t launch_efield(bool dbl, int X, int Y, int Z, double bx, double by, do
   return hipGetLastError();
 }
 
+// rows per workgroup of k_conv_x4: about 512 four-output items
+static int conv_x4_rows(int X) { return std::max(1, 512 / (X / 4)); }
+
+bool conv_pass_ok(bool dbl, int pass, int X, int Y, int Z, int R) {
+  const size_t ts = dbl ? 8 : 4, nt = (2 * (size_t)R + 4) & ~(size_t)3, lim = 64 * 1024;
+  const bool small = (long long)X * Y * Z < (1ll << 31);
+  if (pass == 0)
+    return (R == 5 && small && X % 4 == 0 && X >= 8 && ts * conv_x4_rows(X) * (X + 16) <= lim) ||
+           ts * (nt + 4 * (X + 2 * (size_t)R)) <= lim;
+  return (R == 5 && small) ||
+         (ts * (nt + (kConvTJ + 2 * (size_t)R) * 64) <= lim && (pass == 1 ? Z : Y) <= 65535);
+}
+
 hipError_t launch_conv_pass(bool dbl, int pass, int X, int Y, int Z, int R, const void* taps,
                             const void* in, void* out, hipStream_t s, bool sym) {
   const size_t ts = dbl ? 8 : 4;
@@ -1321,8 +1334,7 @@ hipError_t launch_conv_pass(bool dbl, int pass, int X, int Y, int Z, int R, cons
     const size_t vb = 4 * ts;
     if (R == 5 && X % 4 == 0 && X >= 8 && (uintptr_t)in % vb == 0 && (uintptr_t)out % vb == 0 &&
         (size_t)X * nrows < (1ull << 31)) {
-      // about 512 four-output items per workgroup
-      const int RW = std::max(1, 512 / (X / 4));
+      const int RW = conv_x4_rows(X);
       const size_t lds = ts * (size_t)RW * (X + 16);
       if (lds <= 64 * 1024) {
         const unsigned g = (unsigned)((nrows + RW - 1) / RW);
@@ -1443,21 +1455,14 @@ static void useries_t(int X, int Y, int Z, const UTaps* taps, const double* xtap
 hipError_t launch_useries(bool dbl, int X, int Y, int Z, const UTaps* taps, const double* xtap,
                           int Rx, const void* rho, void* a, void* b, void* phi, bool add,
                           hipStream_t s) {
-  // the radii and grids that launch_conv_pass takes
-  const size_t ts = dbl ? 8 : 4, nx = (2 * (size_t)Rx + 4) & ~(size_t)3;
-  if (ts * (nx + 4 * (X + 2 * (size_t)Rx)) > 64 * 1024) return hipErrorInvalidConfiguration;
-  for (int pass = 0; pass < 2; pass++)
-    for (int k = 0; k < taps[pass].nterm; k++) {
-      const size_t R = (size_t)taps[pass].R[k], nt = (2 * R + 4) & ~(size_t)3;
-      if (ts * (nt + (kConvTJ + 2 * R) * 64) > 64 * 1024) return hipErrorInvalidConfiguration;
-    }
+  // one row with its halos, which is less than conv_pass_ok allows a term
+  if ((dbl ? 8 : 4) * (X + 2 * (size_t)Rx) > 64 * 1024) return hipErrorInvalidConfiguration;
   if (dbl)
     useries_t<double>(X, Y, Z, taps, xtap, Rx, rho, a, b, phi, add, s);
   else
     useries_t<float>(X, Y, Z, taps, xtap, Rx, rho, a, b, phi, add, s);
   return hipGetLastError();
 }
-
 
 // ---------------------------------------------------------------------------
 // Batched independent systems: the k-pass over every system's half spectrum

@@ -434,6 +434,9 @@ hipError_t launch_conv_pass(bool dbl, int pass, int X, int Y, int Z, int R,
                             const void* taps, const void* in, void* out,
                             hipStream_t s, bool sym = false);
 
+// the grids and radii that launch_conv_pass takes (allocations aligned)
+bool conv_pass_ok(bool dbl, int pass, int X, int Y, int Z, int R);
+
 // u-series potential: phi (+)= sum over up to kUTerms terms of the separable
 // Gaussians rho * x * y * z, sums in FP64.  taps[0] / taps[1]: y / z taps
 // (device, tap[k][-(kUTile-1) .. 2R + 2 kUTile) with zeros outside [0, 2R],

@@ -124,6 +124,32 @@ def test_gseu_chunks_and_ragged_grids(N, b, dims, h):
         assert rel(host(g.getPhi()), phi) <= TOL
 
 
+@pytest.mark.parametrize("dt,X", [(F32, 4096), (F32, 4072), (F64, 2048)], ids=["F32", "F32-4072", "F64"])
+def test_gseu_long_rows(dt, X):
+    """Rows near and past the length from which only a radius of five cells is
+    taken: one term of that radius against the oracle; a second, wider term is
+    refused past it and taken below."""
+    dims = (X, 16, 20)
+    box = tuple(1.0 * m for m in dims)
+    x = systems.water_box(60, 1.0, seed=3, wrap=False)
+    x[:, :3] *= np.array(box)
+    xd = dev(x, dt)
+    xr = xd.double().cpu().numpy()
+    p = orc.Params(dims, box, 2.12)
+    e, f, phi = orc.gseu_step(p, 1, 1.3, xr)
+    o = api.CpuGSEu(dt, dt, 1, 1.3, *dims, 2.12, 0.4, 3.0, 3.0, *box).step(xd, force=True)
+    tol = TOL if dt == F64 else 1e-5
+    assert abs(float(host(o["energy"])[0]) - e) <= tol * abs(e)
+    assert orc.erms(f, host(o["force"]).T) <= tol
+    two = api.CpuGSEu(dt, dt, 2, 1.3, *dims, 2.12, 0.4, 3.0, 3.0, *box)
+    two.spreadCharge1(len(x), xd)
+    if X == 4072:
+        two.solvePoisson()
+    else:
+        with pytest.raises(api._lib.GSEError):
+            two.solvePoisson()
+
+
 def test_gseu_gser_fp32_water():
     xyzq, L, M, s = systems.make("water_3k_M32")
     x32 = dev(xyzq, F32)

@@ -1073,46 +1073,69 @@ __global__ void __launch_bounds__(256)
 // pass reads each row once and writes one grid per term, the y pass convolves
 // those, and the z pass adds the terms' columns into one potential.  One
 // convolution per term with its scaling and adding as passes of their own
-// took 12 + 8 launches and 115 us for four terms at 80^3; these take 11.4 + 10.7
-// + 13.2 us.
+// took 12 + 8 launches and 115 us for four terms at 80^3; these take 10.9 + 8.7
+// + 12.6 us.  One term of radius 5 on 200^3 (FP32, the least favourable: the
+// convolutions of that radius are unrolled): 63 us either way.
 // Sums run in FP64 for both types (one FP64 multiply-add per tap, where a
 // compensated 32-bit sum takes four operations) and are rounded once.  Taps
 // beyond a term's radius are zeros, which is exact here because the spread's
 // grids hold finite values only.
 // ---------------------------------------------------------------------------
-// x pass: RW rows per workgroup with their periodic halo in LDS, one cell per
-// thread and iteration, all terms from the same LDS read; taps [2R+1][kUTerms]
-template <typename T>
+// x pass: RW rows per workgroup with their periodic halo in LDS, four cells per
+// thread and iteration, all NT terms from the same LDS read; taps
+// [2R+1][kUTerms]
+template <typename T, int NT>
 __global__ void __launch_bounds__(256)
-    k_useries_x(int X, int nrows, int RW, int R, int nterm, const double* __restrict__ taps,
+    k_useries_x(int X, int nrows, int RW, int R, const double* __restrict__ taps,
                 const T* __restrict__ in, T* __restrict__ out, size_t np) {
   extern __shared__ __align__(16) unsigned char conv_smem[];
   T* lds = (T*)conv_smem;
   const int P = X + 2 * R;
   const int r0 = blockIdx.x * RW, rw = min(RW, nrows - r0);
-  for (int e = threadIdx.x; e < rw * P; e += 256) {
-    const int row = e / P, x = e - row * P - R;
-    lds[e] = in[(size_t)(r0 + row) * X + wrap_small(x, X)];
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e < rw * X; e += 256) {
-    const int row = e / X;
-    const T* w = lds + row * P + (e - row * X);
-    double acc[kUTerms] = {};
-#pragma unroll 4
-    for (int d = 0; d <= 2 * R; d++) {
-      const double v = (double)w[d];
+  // quotients of e < 2^15 as float products (exact: (e + 1/2) / d lies at
+  // least 1/(2d) from a whole number), a third of the instructions per cell
+  const float inv_p = 1.0f / (float)P, inv_x = 1.0f / (float)X;
+  for (int e0 = threadIdx.x; e0 < rw * P; e0 += 4 * 256) {
+    T v[4];
 #pragma unroll
-      for (int j = 0; j < kUTerms; j++)
-        acc[j] = __builtin_fma(taps[d * kUTerms + j], v, acc[j]);
+    for (int u = 0; u < 4; u++) {
+      const int e = min(e0 + 256 * u, rw * P - 1), row = (int)(((float)e + 0.5f) * inv_p);
+      v[u] = in[(size_t)(r0 + row) * X + wrap_small(e - row * P - R, X)];
     }
 #pragma unroll
-    for (int j = 0; j < kUTerms; j++)
-      if (j < nterm) out[j * np + (size_t)r0 * X + e] = (T)acc[j];
+    for (int u = 0; u < 4; u++)
+      if (e0 + 256 * u < rw * P) lds[e0 + 256 * u] = v[u];
+  }
+  __syncthreads();
+  // four cells a thread share each tap's scalar load
+  const int n = rw * X;
+  for (int e0 = threadIdx.x; e0 < n; e0 += 4 * 256) {
+    const T* w[4];
+    double acc[4][NT] = {};
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int e = min(e0 + 256 * u, n - 1), row = (int)(((float)e + 0.5f) * inv_x);
+      w[u] = lds + row * P + (e - row * X);
+    }
+#pragma unroll 4
+    for (int d = 0; d <= 2 * R; d++)
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const double v = (double)w[u][d];
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+          acc[u][j] = __builtin_fma(taps[d * kUTerms + j], v, acc[u][j]);
+      }
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+#pragma unroll
+      for (int j = 0; j < NT; j++)
+        if (e0 + 256 * u < n) out[j * np + (size_t)r0 * X + e0 + 256 * u] = (T)acc[u][j];
   }
 }
 
-// TJ consecutive outputs of one column: inputs j .. along an axis of length N
+// TJ consecutive outputs of one column (8: 2.25 loads an output at radius 5;
+// with 4 outputs the y and the z pass took 22 us each on 200^3, 18 with 8): inputs j .. along an axis of length N
 // and stride S from the column's first element; tap[-(TJ-1) .. 2R + 2TJ) with
 // zeros outside [0, 2R].  j is wave-uniform, its periodic wrap scalar work.
 template <typename T, int TJ>
@@ -1436,8 +1459,12 @@ static void useries_t(int X, int Y, int Z, const UTaps* taps, const double* xtap
                       const void* rho, void* a, void* b, void* phi, bool add, hipStream_t s) {
   const size_t np = (size_t)X * Y * Z;
   const int nrows = Y * Z, RW = useries_rows(sizeof(T), X, Rx), nt = taps[0].nterm;
-  k_useries_x<T><<<(nrows + RW - 1) / RW, 256, sizeof(T) * RW * (X + 2 * (size_t)Rx), s>>>(
-      X, nrows, RW, Rx, nt, xtap, (const T*)rho, (T*)a, np);
+  const auto kx = nt == 1   ? k_useries_x<T, 1>
+                  : nt == 2 ? k_useries_x<T, 2>
+                  : nt == 3 ? k_useries_x<T, 3>
+                            : k_useries_x<T, 4>;
+  kx<<<(nrows + RW - 1) / RW, 256, sizeof(T) * RW * (X + 2 * (size_t)Rx), s>>>(
+      X, nrows, RW, Rx, xtap, (const T*)rho, (T*)a, np);
   for (int pass = 1; pass < 3; pass++) {
     const int N = pass == 1 ? Y : Z, C = pass == 1 ? X * Z : X * Y, cw = pass == 1 ? X : X * Y;
     const long long S = pass == 1 ? X : (long long)X * Y, cs = pass == 1 ? (long long)X * Y : 0;

@@ -442,7 +442,7 @@ bool conv_pass_ok(bool dbl, int pass, int X, int Y, int Z, int R);
 // (device, tap[k][-(kUTile-1) .. 2R + 2 kUTile) with zeros outside [0, 2R],
 // the terms' factors in the z taps); xtap: [2Rx+1][kUTerms], zeros where a
 // term is narrower; a, b: kUTerms grids each.
-constexpr int kUTerms = 4, kUTile = 4;
+constexpr int kUTerms = 4, kUTile = 8;
 struct UTaps {
   int nterm;
   int R[kUTerms];

@@ -1134,10 +1134,11 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// TJ consecutive outputs of one column (8: 2.25 loads an output at radius 5;
-// with 4 outputs the y and the z pass took 22 us each on 200^3, 18 with 8): inputs j .. along an axis of length N
+// TJ consecutive outputs of one column: inputs j .. along an axis of length N
 // and stride S from the column's first element; tap[-(TJ-1) .. 2R + 2TJ) with
 // zeros outside [0, 2R].  j is wave-uniform, its periodic wrap scalar work.
+// Eight outputs take three loads each at radius 5, four take four: the y and
+// the z pass of one term on 200^3 took 18 us each with eight, 22 with four.
 template <typename T, int TJ>
 __device__ __forceinline__ void useries_col(const T* __restrict__ col, long long S, int N, int j,
                                             int R, const double* __restrict__ tap,

@@ -2216,11 +2216,17 @@ gse_status_t gse_ewald_direct_calc_force_energy(gse_ewald_direct_t h, int n, con
   GSECHK(h->starts.ensure(sizeof(int) * (c.ncell + 1)));
   GSECHK(h->partials.ensure(sizeof(double) * n1));
   GSECHK(h->q2.ensure(sizeof(double) * kEwCountBlocks));
-  if (!h->erfcx.p) {
-    GSECHK(h->erfcx.ensure(ew_erfcx_bytes()));
-    HIPCHK(hipMemcpy(h->erfcx.p, ew_erfcx_table(), ew_erfcx_bytes(), hipMemcpyHostToDevice));
-  }
   hipStream_t s = h->stream;
+  if (!h->erfcx.p) {  // once, on the handle's stream; kept only when the copy is complete
+    GSECHK(h->erfcx.ensure(ew_erfcx_bytes()));
+    hipError_t e = hipMemcpyAsync(h->erfcx.p, ew_erfcx_table(), ew_erfcx_bytes(),
+                                  hipMemcpyHostToDevice, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e != hipSuccess) {
+      h->erfcx.release();
+      return fail(GSE_ERROR_HIP, "erfcx table upload failed: %s", hipGetErrorString(e));
+    }
+  }
   HIPCHK(launch_ew_cells(xyzq, n, c, h->rcut, h->cell_of.as<int>(), h->rank.as<int>(),
                          h->counts.as<int>(), h->starts.as<int>(), h->tmp.as<int>(),
                          h->sidx.as<int>(), h->sx.p, h->sf.p, h->q2.as<double>(), s));

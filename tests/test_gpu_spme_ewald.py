@@ -247,6 +247,19 @@ def test_spme_without_bricks(dt, order):
         api.set_tuning(spread_flush=1)
 
 
+@pytest.mark.parametrize("dims", [(256, 256, 128), (264, 256, 128)], ids=["16384", "16896"])
+def test_spme_many_bins(dims):
+    """The most bins whose slots are claimed a workgroup at a time, and more."""
+    box = tuple(1.03 * m for m in dims)
+    n = 20000
+    x = spme_uneven(n, box, 2)
+    pm = api.CudaPMERecip(F64, F64, *dims, 4)
+    for _ in range(2):
+        pm.spread_charge(dev(x), n, box)
+        q = orc.pme_spread(dims, 4, x[np.isfinite(x).all(axis=1)], box)
+        assert rel(host(pm.grid()).ravel(), np.asarray(q).ravel()) <= TOL
+
+
 def test_spme_bad_arguments():
     with pytest.raises(api._lib.GSEError):
         api.CudaPMERecip(F64, F64, 16, 16, 16, 5)
@@ -303,7 +316,7 @@ def test_ewald_direct_fp64(case):
 EW_EDGES = [((0.7, 0.7, 0.7), 2, 1.0), ((0.7, 1.6, 3.3), 65, 1.0), ((2.4, 2.4, 2.4), 200, 1.0),
             ((2.51, 2.99, 3.0), 200, 1.0), ((3.2, 2.4, 3.1), 129, 1.0), ((5.0, 0.9, 2.5), 257, 1.0),
             ((40.0, 3.0, 3.0), 64, 1.0), ((4.0, 4.0, 4.0), 1, 1.0),
-            # erfc far out: rcut / (sqrt(2) sigma) = 8.8 and 35
+            # narrow Gaussians: rcut / (sqrt(2) sigma) = 17.7 and 70.7
             ((3.0, 3.5, 4.0), 300, 0.08), ((3.0, 3.0, 3.0), 150, 0.02)]
 
 
@@ -311,10 +324,12 @@ EW_EDGES = [((0.7, 0.7, 0.7), 2, 1.0), ((0.7, 1.6, 3.3), 65, 1.0), ((2.4, 2.4, 2
 def test_ewald_direct_cell_edges(edges, n, width):
     """The direct sum where the candidate ranges change form, against the
     oracle: coordinates on box faces and several boxes outside, six
-    exclusions per atom, and Gaussian widths down to rcut/50.  A pair term is
+    exclusions per atom, and Gaussian widths down to rcut/100.  A pair term is
     a dozen FP64 roundings and the sums run over at most n terms, so a
     component is off by less than (12 + n) 2^-53 of the sum of its terms'
-    magnitudes, bounded here by n times the largest pair force."""
+    magnitudes, bounded here by n times the largest pair force.  (Far out in
+    erfc the pairs are too weak to be seen beside that one:
+    test_ewald_direct_pair_far_out looks at them one by one.)"""
     rcut = 6.0
     box = tuple(rcut * e for e in edges)
     rng = np.random.default_rng(n)
@@ -338,10 +353,55 @@ def test_ewald_direct_cell_edges(edges, n, width):
     f = torch.zeros((3, n), dtype=F64, device="cuda")
     eg = d.calcForceEnergy(n, dev(x), f[0], f[1], f[2])
     fg = host(f).T
-    scale = max(np.max(np.abs(g)), 1e-300)
+    excl = {(i - 1, j) for j in range(n) for i in nb[(ib[j - 1] if j else 0):ib[j]]}
+    scale = 1e-300
+    for j in range(n - 1):
+        d = x[j + 1:, :3] - x[j, :3]
+        d -= np.array(box) * np.rint(d / np.array(box))
+        r = np.sqrt((d * d).sum(axis=1))
+        for i in np.flatnonzero((r < rcut) & (r > 0)):
+            if (i + j + 1, j) not in excl:
+                u = r[i] / (math.sqrt(2.0) * sigma)
+                w = (2.0 / math.sqrt(math.pi) * u * math.exp(-u * u) + math.erfc(u)) / r[i] ** 2
+                scale = max(scale, 332.0716 * w * abs(x[j, 3] * x[i + j + 1, 3]))
     print(f"E {e:.12e} gpu {eg:.12e} max dF/F {np.max(np.abs(fg - g)) / scale:.1e}", flush=True)
     assert np.max(np.abs(fg - g)) <= (12 + n) * n * 2.0 ** -53 * scale
     assert abs(eg - e) <= (12 + n) * 2.0 ** -53 * n * max(abs(e), 332.0716 / sigma)
+
+
+@pytest.mark.parametrize("u", [1e-3, 0.1, 0.2499, 0.25, 0.2501, 1.9941, 3.99, 7.99, 8.0, 8.01, 9.5,
+                               15.0, 20.0, 25.0, 26.4])
+def test_ewald_direct_pair_far_out(u):
+    """One pair at u = r / (sqrt(2) sigma), each force relative to itself: the
+    erfcx intervals on both sides of 8 and out to where erfc leaves the normal
+    range.  exp(-u^2) and the oracle's erfc(u) turn the roundings of their
+    arguments (three here, two and a half of twice the weight there) into at
+    most 3 + 5 of u^2 2^-53; the rest is about twenty roundings."""
+    r = 4.7
+    sigma = r / (math.sqrt(2.0) * u)
+    x = np.array([[1.0, 2.0, 3.0, 0.7], [1.0 + 0.48 * r, 2.0 - 0.6 * r, 3.0 + 0.64 * r, -0.3]])
+    box = (14.0, 15.0, 16.0)
+    e, g = orc.ewald_direct(sigma, 6.0, box, x)
+    f = torch.zeros((3, 2), dtype=F64, device="cuda")
+    eg = api.CpuEwaldDirect(sigma, 6.0, *box).calcForceEnergy(2, dev(x), f[0], f[1], f[2])
+    fg = host(f).T
+    err = np.max(np.abs(fg - g) / np.abs(g))
+    tol = (10 + 4 * u * u) * 2.0 ** -52
+    print(f"u {u}: {err:.1e} of {tol:.1e}, force {np.abs(g).max():.1e}", flush=True)
+    assert np.min(np.abs(g)) > 1e-307 and err <= tol
+    assert abs(eg - e) <= (10 + 4 * u * u) * 2.0 ** -52 * (abs(e) + 332.0716 / sigma)
+
+
+@pytest.mark.parametrize("u", [26.9, 27.0, 27.1, 30.0, 1e3, 1e8])
+def test_ewald_direct_pair_past_underflow(u):
+    """Where erfc leaves the normal range the force is that small, not garbage."""
+    x = np.array([[1.0, 2.0, 3.0, 0.7], [5.0, 2.0, 3.0, -0.3]])
+    f = torch.full((3, 2), 7.0, dtype=F64, device="cuda")
+    sigma = 4.0 / (math.sqrt(2.0) * u)
+    e = api.CpuEwaldDirect(sigma, 6.0, 14.0, 15.0, 16.0).calcForceEnergy(2, dev(x), f[0], f[1], f[2])
+    assert np.max(np.abs(host(f))) <= 1e-300
+    own = -332.0716 * (0.7 ** 2 + 0.3 ** 2) / math.sqrt(2.0 * math.pi * sigma ** 2)
+    assert abs(e - own) <= 1e-14 * abs(own)
 
 
 def test_total_electrostatics_like_test48k():

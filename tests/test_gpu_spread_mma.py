@@ -116,8 +116,12 @@ def test_mma_spread_bin_counts(extra):
     """Bins around one and two matrix steps, past the tables, and past the
     exact class sums, on a grid with 2- and 7-cell last bins: within FP32 accuracy of
     the oracle and bit-identical in any order.  A value is off by the
-    roundings of its bricks (half of 2^-30 of the bin's bound of extra
-    charges, at most 27 bricks) and by 2^-23 of each charge's factors."""
+    roundings of its bricks (at most 27; each half a unit of 2^-30 of the power
+    of two above its charges' sum, so of at most twice the n charges) and by
+    its charges' factors: each of three exponentials is off by up to two units
+    of 2^-24, its argument's rounding by less than one more, so a charge by
+    less than 9 2^-24 < 2^-20 and by a third of that as a root mean square,
+    and the n charges' independent errors add up as the root of n."""
     rng = np.random.default_rng(extra)
     dims, box = (26, 31, 40), (26.0, 31.0, 40.0)
     n = 400 + extra
@@ -194,6 +198,26 @@ def test_mma_spread_giant_bin_takes_the_per_contribution_path():
     r0, _ = spread32(xyzq, p, False)
     assert lay1["spread"] == "mma"
     assert torch.equal(r1, r0)
+
+
+def test_mma_default_rule_by_occupancy():
+    """The default picks the matrix cores from 24 to 72 charges a bin on
+    average; one handle crosses both limits in both directions, and its grids
+    equal the oracle's throughout."""
+    dims, L = (24, 24, 24), 24.0
+    p = orc.Params(dims, (L,) * 3, 2.12)
+    nb = 27
+    rng = np.random.default_rng(8)
+    xyzq = rng.random((72 * nb + 1, 4)) * np.array([L, L, L, 1.0]) - np.array([0, 0, 0, 0.5])
+    assert api.get_tuning()["spread_mma"] == 2
+    g = api.CpuGaussCharge(F32, F32, *dims)
+    rho = torch.zeros((24, 24, 24), dtype=F32, device=DEV)
+    for n, want in ((24 * nb - 1, "lds_atomic"), (24 * nb, "mma"), (72 * nb + 1, "lds_atomic"),
+                    (72 * nb, "mma"), (24 * nb - 1, "lds_atomic"), (40 * nb, "mma")):
+        g.spreadChargeToGrid(p.sigma1, p.rcut1, n, to_dev(xyzq[:n]), *p.box, rho)
+        assert g.layout()["spread"] == want and g.layout()["nbins"] == nb, n
+        ref = orc.spread(p.dims, p.sigma1, p.rcut1, xyzq[:n].astype(np.float32).astype(np.float64), p.box)
+        assert rel(host(rho), ref) <= 2e-6, n
 
 
 def test_mma_gsek_step_fp32_force_rms():

@@ -985,8 +985,8 @@ __global__ __launch_bounds__(1024) void k_ew_finalize(const double* __restrict__
 }
 
 void ew_cells_make(const double* box, double rcut, int n, EwCells* c) {
-  // about four cells per particle at most, so that a sparse box does not
-  // spend its time on empty cells
+  // about eight cells per particle at most (16 for one), so that a sparse box
+  // does not spend its time on empty cells
   const int cap = std::max(2, std::min(64, (int)std::cbrt(4.0 * n)));
   c->ncell = 1;
   for (int a = 0; a < 3; a++) {

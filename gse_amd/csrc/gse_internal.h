@@ -504,7 +504,7 @@ struct EwPair {
 };
 constexpr int kEwCountBlocks = 256;
 // cells of n particles: rcut/4 along x, rcut/2 along y and z, at most about
-// four per particle
+// eight per particle
 void ew_cells_make(const double* box, double rcut, int n, EwCells* c);
 void ew_filter_make(const EwCells& c, EwPair* p);
 // cell lists: counts [ncell], starts [ncell + 1], cell_of/rank/tmp/sidx [n],

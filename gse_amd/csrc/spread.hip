@@ -1156,9 +1156,8 @@ __device__ __forceinline__ void mma_giant_bin(const SpreadArgs& a,
   for (int i = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); i < cnt; i += WAVES)
     spread_one_global<float>(a.g, a.inv2s2, a.pref, S, 0, a.pref1, slots[i], grid64, shift);
 }
-__device__ __forceinline__ bool mma_giant(int call, int cap_bin) {
-  return call > kMmaMaxCall || call > cap_bin + kMmaOvfList;
-}
+static_assert(kMmaMaxCall <= kMmaOvfList, "a bin's overflow particles fit its list");
+__device__ __forceinline__ bool mma_giant(int call) { return call > kMmaMaxCall; }
 
 // One bin: the brick of its `call` particles (cnt in slots, the rest on the
 // overflow list) and its shift, or, for a giant bin, its slots' particles in
@@ -1176,7 +1175,7 @@ __device__ __forceinline__ void mma_bin(const SpreadArgs& a, MmaLds& m, int bin,
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ebin = fixed_exponent_bin(qbits, call, a.pref_bound);
   const int shift = eg > ebin ? eg - ebin : 0;
-  const bool giant = mma_giant(call, a.cap_bin);
+  const bool giant = mma_giant(call);
   if (tid == 0) bshift[bin] = giant ? -1 : shift;
   if (giant) {
     mma_giant_bin<WAVES>(a, slots, cnt, eg, shift, grid64);
@@ -1334,7 +1333,7 @@ __global__ void __launch_bounds__(64 * WAVES, 4)
     const int gw = __builtin_amdgcn_readfirstlane(w * WAVES + (int)(threadIdx.x >> 6));
     for (int k = gw; k < st.overflow; k += kOverflowWG * WAVES) {
       const V4<float> p = xyzq[ovf[k]];
-      if (mma_giant(counts[home_bin<float>(a.g, a.b, p)], a.cap_bin))
+      if (mma_giant(counts[home_bin<float>(a.g, a.b, p)]))
         spread_overflow<float, unsigned>(a, eg, st.qmax_bits, counts, p, grid64);
     }
     return;

@@ -991,17 +991,18 @@ __global__ void __launch_bounds__(BS, BS == 512 ? 6 : 1)
 // into the same brick, and the int64 total is rounded once to the bin's
 // int32 scale 2^(e - shift), the scale and shift of the LDS-atomic path.
 //
-// Layout.  Four waves (eight on small grids) share the bin's 25 row tiles (25 x 16 = 20 x 20 points
-// exactly).  The factors go to LDS once as tables over (axis position,
-// particle), zero outside a particle's window, one lane per particle; a lane
-// then forms its row's A values of 16 consecutive particles from eight
-// 16-byte table reads and holds them as matrix operands without another trip
-// through LDS, and the results go from the accumulators to memory.  There is
-// no brick in LDS, so four workgroups share a CU and the 1000 bins of an 80^3
-// grid run at once.  The bound is VALU issue: seven instructions per A value,
-// eight per brick cell, and the chain from the counts to the tables.  Rows of the x and y tables are 132 floats apart: the
+// Layout.  Four waves (eight on small grids) share the bin's 25 row tiles
+// (25 x 16 = 20 x 20 points exactly).  The factors go to LDS once as tables
+// over (axis position, particle), zero outside a particle's window, one lane
+// per particle; a lane then forms its row's A values of 16 consecutive
+// particles from eight 16-byte table reads and holds them as matrix operands
+// without another trip through LDS, and the results go from the accumulators
+// to memory.  There is no brick in LDS, so four workgroups share a CU and the
+// 1000 bins of an 80^3 grid run at once.  The bound is VALU issue: seven
+// instructions per A value, eight per brick cell, and the chain from the
+// counts to the tables.  Rows of the x and y tables are 132 floats apart: the
 // 16 x positions a 16-lane group reads fall on distinct 16-byte bank groups.
-// Measured at 80^3 / 48,000 charges and 216^3 / 1,000,002: 24.8 and 317 us,
+// Measured at 80^3 / 48,000 charges and 216^3 / 1,000,002: 23.0 and 282 us,
 // against 32.4 and 437 us with LDS atomics; grid error against the FP64 oracle
 // 3.3e-7 of the largest value, against 1.34e-6.
 // Operand layouts: A lane l -> row l % 16, B lane l -> column l % 16, and
@@ -1363,14 +1364,15 @@ bool spread_mma_ok(bool dbl, const Geom& g, const BinShape& b, bool normalize, b
   // matrix path the same from 1 to 64 charges and little more to 128, the LDS
   // path in proportion to them; a bin past 128 builds the tables several times,
   // and the launch waits for it.
-  // Measured, LDS / matrix us: 80^3 with 18 a bin 22.1 / 24.7, 24 25.4 / 25.0,
-  // 36 29.7 / 25.4, 48 34.8 / 26.0, 72 44.7 / 29.1, 96 54.0 / 61.0; 160^3 with
-  // 18 104 / 118, 24 115 / 118, 36 143 / 118, 72 242 / 160; 40^3 with 18 13.8 /
-  // 12.9, 72 23.8 / 15.5, 96 26.9 / 30.7.  The mean also decides for boxes filled
-  // in part, where it says less: the whole call at 80^3 with half the box
-  // empty takes 71.4 / 46.6 us at 96 charges in a filled bin and 95.2 / 81.3 at
-  // 144; 160^3 561 / 470 at 144; with more than two thirds empty the LDS path's
-  // overflow costs over 1 ms.
+  // Measured, the whole spread call with LDS / matrix cores in us: 80^3 with 12
+  // a bin 36.1 / 38.3, 18 38.8 / 38.5, 24 39.9 / 37.9, 48 50.7 / 39.0, 72
+  // 60.4 / 47.8, 96 72.2 / 49.0; 160^3 with 24 195 / 175, 72 358 / 265; 24^3
+  // with 24 20.8 / 18.9, 72 28.1 / 22.4.  Below 24 the difference is within 5 %;
+  // 72 keeps all but a few bins of a box of water within one set of tables.
+  // The mean also decides for boxes filled in part, where it says less: at 80^3
+  // with half the box empty the call takes 71.4 / 46.6 us at 96 charges in a
+  // filled bin and 95.2 / 81.3 at 144; 160^3 561 / 470 at 144; with more than
+  // two thirds empty the LDS path's overflow costs over 1 ms.
   const int knob = tuning().spread_mma;
   return knob == 1 || (knob == 2 && n >= 24LL * b.nbins && n <= 72LL * b.nbins);
 }
@@ -2493,7 +2495,8 @@ static hipError_t spread_t(const Geom& g, const BinShape& b, double sigma, bool 
     a.nwg_bins = ((b.nbins + 7) / 8) * 8;
     // eight waves a bin while every bin has a CU's matrix cores to itself or
     // shares them with one other: the chain of row tiles sets the time there
-    // (32^3: 16.7 against 12.4 us, 54 x 63 x 50: 21.2 against 19.0); four give more bins at once beyond
+    // (32^3: 16.7 us with four and 12.4 with eight when chosen, 54 x 63 x 50:
+    // 21.2 and 19.0); four give more bins at once beyond
     const bool few = b.nbins <= 512;
     (few ? k_spread_mma<8> : k_spread_mma<4>)<<<(unsigned)a.nwg_bins + kOverflowWG, few ? 512 : 256,
                                                0, s>>>(

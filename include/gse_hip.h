@@ -546,14 +546,17 @@ GSE_API gse_status_t gse_batch_autotune(gse_batch_t h, const void* xyzq, int rep
 typedef struct gse_pme_recip_s* gse_pme_recip_t;
 
 /* CudaPMERecip.h:143-145  CudaPMERecip(nfftx, nffty, nfftz, order, BOX, 1, 0, ...);
- * order 4, 6 or 8; every dimension at least the order. */
+ * order 4, 6 or 8; every dimension at least the order.  Device memory beside the
+ * grids: 21, 38 or 53 bytes a grid cell (order 4, 6, 8) for the spread's bricks,
+ * which it does without where they do not fit. */
 GSE_API gse_status_t gse_pme_recip_create(gse_pme_recip_t* out, gse_dtype_t at, gse_dtype_t ct,
                                           int nfftx, int nffty, int nfftz, int order);
 GSE_API gse_status_t gse_pme_recip_destroy(gse_pme_recip_t h);
 /* CudaPMERecip.h:152 */
 GSE_API gse_status_t gse_pme_recip_set_stream(gse_pme_recip_t h, void* hip_stream);
 /* CudaPMERecip.h:155  spread_charge(xyzq, ncoord, recip): B-spline spread
- * of device particles {x, y, z, q} (CT) into the handle's grid */
+ * of device particles {x, y, z, q} (CT) into the handle's grid.  May be captured
+ * into a HIP graph, which the handle must outlive */
 GSE_API gse_status_t gse_pme_recip_spread_charge(gse_pme_recip_t h, const void* xyzq, int ncoord,
                                                  const double* recip);
 /* CudaPMERecip.h:173-174  r2c_fft(), c2r_fft() on the handle's grid */
